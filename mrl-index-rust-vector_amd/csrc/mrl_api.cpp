@@ -72,7 +72,7 @@ struct mrl_ctx {
   int s4_policy = MRL_S4_BOUND_AUTO;  // mrl_ctx_set_s4_bound
   std::vector<ProfRecord> prof;       // recorded, not yet collected
   std::vector<hipEvent_t> event_pool; // reusable events
-  uint32_t* d_crc = nullptr;          // encoder CRC tables: [256] byte table, then [64][32] carry map
+  uint32_t* d_crc = nullptr;          // encoder CRC tables: [4][256] slicing tables, then [64][32] carry map
   uint8_t* d_evict = nullptr;         // cache-eviction buffer (mrl_ctx_evict_caches), zero-filled
   uint64_t evict_bytes = 0;
   uint32_t crc_const = 0;
@@ -2846,6 +2846,30 @@ extern "C" int mrl_encode_corpus_clustered(const float* matrix, uint64_t n, uint
 }
 
 
+// The largest float in [a, b) nearer to a than to b, ties to a (nearest_centroid, eden.rs:58-71, between two
+// neighbouring levels): fl(t - a) grows and fl(b - t) falls with t, so the predicate flips once.
+static float level_limit(float a, float b) {
+  auto order = [](float f) {
+    int32_t i;
+    memcpy(&i, &f, 4);
+    return i < 0 ? (int32_t)(0x80000000u - (uint32_t)i) : i;
+  };
+  auto value = [](int32_t i) {
+    if (i < 0) i = (int32_t)(0x80000000u - (uint32_t)i);
+    float f;
+    memcpy(&f, &i, 4);
+    return f;
+  };
+  int32_t lo = order(a), hi = order(b);  // true at lo, false at hi
+  while (hi - lo > 1) {
+    const int32_t mid = lo + (hi - lo) / 2;
+    const float t = value(mid);
+    if (fabsf(t - a) <= fabsf(b - t)) lo = mid;
+    else hi = mid;
+  }
+  return value(lo);
+}
+
 // CRC-32 tables for the GPU encoder.  raw(c, M) is the reflected CRC register
 // after bytes M starting from register c (no initial or final xor); it is
 // linear in c and M over GF(2), so
@@ -2853,7 +2877,7 @@ extern "C" int mrl_encode_corpus_clustered(const float* matrix, uint64_t n, uint
 // for the 64-byte chunks M_k, with carry(c, L) = raw(c, 0^L) = xor over the
 // set bits i of c of carry(1 << i, L).
 struct CrcTables {
-  uint32_t tab[256 + 64 * 32];
+  uint32_t tab[1024 + 64 * 32];  // slicing tables, then the carry map
   uint32_t konst;
 };
 static const CrcTables& crc_tables() {
@@ -2864,12 +2888,13 @@ static const CrcTables& crc_tables() {
       for (int k = 0; k < 8; ++k) c = (c & 1u) ? (0xEDB88320u ^ (c >> 1)) : (c >> 1);
       r.tab[i] = c;
     }
+    for (uint32_t i = 256; i < 1024; ++i) r.tab[i] = r.tab[r.tab[i - 256] & 0xffu] ^ (r.tab[i - 256] >> 8);
     auto zeros = [&](uint32_t c, uint32_t nbytes) {
       for (uint32_t j = 0; j < nbytes; ++j) c = r.tab[c & 0xffu] ^ (c >> 8);
       return c;
     };
     for (uint32_t k = 0; k < 64; ++k)
-      for (uint32_t i = 0; i < 32; ++i) r.tab[256 + 32 * k + i] = zeros(1u << i, 64u * (63u - k));
+      for (uint32_t i = 0; i < 32; ++i) r.tab[1024 + 32 * k + i] = zeros(1u << i, 64u * (63u - k));
     r.konst = zeros(0xffffffffu, kBlockBytes) ^ 0xffffffffu;
     return r;
   }();
@@ -2894,32 +2919,30 @@ static int encode_device(mrl_ctx* ctx, const float* d_matrix, uint64_t n, uint32
     HIP_TRY(hipMemcpy(ctx->d_crc, t.tab, sizeof(t.tab), hipMemcpyHostToDevice));
     ctx->crc_const = t.konst;
   }
-  float* d_means = nullptr;
-  if (hipMalloc(&d_means, 192 * sizeof(float)) != hipSuccess) return fail(MRL_ERR_OUT_OF_MEMORY, "fit means");
-  hipError_t e = hipSuccess;
-  if (eden) e = hipMemcpy(d_means, eden->mean, 64 * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess && eden_mid) e = hipMemcpy(d_means + 64, eden_mid->mean, 128 * sizeof(float), hipMemcpyHostToDevice);
   EncodeArgs a{};
   a.x = d_matrix;
   a.n = n;
   a.dims = dims;
   a.cluster = d_cluster;
   a.source = default_source;
-  a.eden_mean = eden ? d_means : nullptr;
+  a.eden = eden ? 1 : 0;
+  a.mid = eden_mid ? 1 : 0;
+  if (eden) memcpy(a.means, eden->mean, 64 * sizeof(float));
+  if (eden_mid) memcpy(a.means + 64, eden_mid->mean, 128 * sizeof(float));
   a.eden_seed = eden ? eden->seed : 0;
-  a.mid_mean = eden_mid ? d_means + 64 : nullptr;
   a.mid_seed = eden_mid ? eden_mid->seed : 0;
+  for (int l = 0; l < 15; ++l) a.level_max[l] = level_limit(ctx->consts.eden_codebook[l], ctx->consts.eden_codebook[l + 1]);
+  a.mid_level_max = level_limit(ctx->consts.eden_mid_codebook[0], ctx->consts.eden_mid_codebook[1]);
   a.crc_tab = ctx->d_crc;
-  a.crc_zt = ctx->d_crc + 256;
+  a.crc_zt = ctx->d_crc + 1024;
   a.crc_const = ctx->crc_const;
   a.c = ctx->consts;
   a.sqrt64 = sqrtf(64.0f);
   a.sqrt128 = sqrtf(128.0f);
   a.out = static_cast<uint8_t*>(d_out_blocks);
   a.n_blocks = (n + 63) / 64;
-  if (e == hipSuccess) e = launch_encode(a, ctx->stream);
+  hipError_t e = launch_encode(a, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  dev_free(d_means);
   if (e != hipSuccess) return fail(MRL_ERR_HIP, std::string("encode: ") + hipGetErrorString(e));
   return MRL_OK;
 }

@@ -363,11 +363,18 @@ struct EncodeArgs {
   uint32_t dims;
   const uint32_t* cluster; // [n] coarse cluster of each row (device) or null: the cluster-grouped convention
   uint32_t source;         // source id of every row
-  const float* eden_mean;  // 64 floats (device) or null: MinMax4 prefix
+  int32_t eden;            // EdenProd prefix (else MinMax4)
+  int32_t mid;             // EdenB1 mid-band (else RaBitQ); needs eden
+  float means[192];        // fit means: prefix 64, mid 128
   uint64_t eden_seed;
-  const float* mid_mean;   // 128 floats (device) or null: RaBitQ mid-band
   uint64_t mid_seed;
-  const uint32_t* crc_tab; // [256] CRC-32 byte table
+  uint64_t eden_signs;     // Rademacher signs of the seeds (bit i set: -1), filled by launch_encode
+  uint64_t mid_signs[2];
+  // nearest_centroid (eden.rs:58-71) as thresholds: level_max[l] is the largest float whose nearest level is at
+  // most l, so the level of z is the number of them below z (a NaN has level 0)
+  float level_max[15];
+  float mid_level_max;
+  const uint32_t* crc_tab; // [4][256] CRC-32 slicing tables: byte i followed by k zero bytes
   const uint32_t* crc_zt;  // [64][32]: register bit i of chunk k carried past the following 64*(63-k) bytes
   uint32_t crc_const;      // CRC of 4096 zero bytes (initial register and final xor folded in)
   PlanConsts c;

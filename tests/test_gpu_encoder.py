@@ -91,3 +91,27 @@ def test_gpu_encoder_benchmark_corpus_slice(device):
     rows = synth.docs(w, 0, 65536)
     gpu, _, _ = _gpu_encode(rows, device, 0, fit)
     assert np.array_equal(gpu, m.encode_corpus(rows, 0, fit))
+
+
+@pytest.mark.parametrize("n,dims,offset", [
+    (64 * 1024 + 64 * 3 + 5, 192, 0),  # more blocks than waves in the grid: every wave's second block; no tail
+    (64 * 1024 + 64 * 3 + 5, 194, 0),  # the same with 4-byte loads (rows not 16-byte aligned), a part piece
+    (64 * 2 + 1, 256, 0),              # one folded tail block
+    (64 * 2 + 1, 256, 1),              # 4-byte loads because of the base address
+    (64 * 3 - 1, 832, 0),              # a whole piece past the folded dims
+    (64 * 3 - 1, 900, 0),              # and a part one
+    (64 * 3 - 1, 837, 3),
+])
+@pytest.mark.parametrize("kind", ["minmax", "eden", "eden_dual"])
+def test_gpu_encoder_pieces_and_alignments(device, n, dims, offset, kind):
+    """Edges of the encoder's 64-dim pieces, both load widths and the block loop: bytes equal the host encoder's."""
+    rng = np.random.default_rng(dims + offset)
+    rows = normalized(rng, n, dims)
+    eden, mid = _fits(rows[:2000], kind)
+    flat = np.concatenate([np.zeros(offset, dtype=np.float32), rows.ravel()])
+    x = m.DeviceBuffer.from_array(flat, device)
+    n_blocks = (n + 63) // 64
+    out = m.DeviceBuffer(n_blocks * 4096, device)
+    m.encode_corpus_device(x.ptr + 4 * offset, n, dims, out.ptr, device, 8, eden, mid)
+    gpu = out.to_array(np.uint8, (n_blocks, 4096))
+    assert np.array_equal(gpu, m.encode_corpus(rows, 8, eden, mid))
