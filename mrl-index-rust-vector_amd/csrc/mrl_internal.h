@@ -351,6 +351,12 @@ struct SelectArgs {
   float* out_scores;
   uint32_t* out_counts;
   unsigned long long* stats;  // [kStatCopies][kStatCount] or null: flagged re-runs are counted here
+  // The outputs above may be host memory mapped for the device (a synchronous
+  // scan's).  stats_sum (then also mapped host memory) gets the counters of
+  // stats_src summed over their copies, complete but for this launch's own
+  // re-run counts (which status holds); null: not asked for.
+  const unsigned long long* stats_src;
+  unsigned long long* stats_sum;
   // Gated re-run: query q is selected only if bit 2 of gate[q] is set
   // (gate is the status array this launch rewrites); null: every query.
   const uint32_t* gate;

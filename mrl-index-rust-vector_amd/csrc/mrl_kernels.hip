@@ -2203,11 +2203,13 @@ __global__ __launch_bounds__(kSelThreads) void k_select(SelectArgs a) {
   }
   }
   const uint32_t keep = m < K ? m : K;
-  auto emit = [&](uint32_t r, uint64_t c) {
-    const uint32_t row = ~(uint32_t)c;
-    a.out_ids[(uint64_t)q * K + r] = ((uint64_t)(row >> 6) << 16) | (uint64_t)(row & 63u);
-    a.out_scores[(uint64_t)q * K + r] = key_score((uint32_t)(c >> 32));
-  };
+  // The sorted entries are collected in LDS and written out in order, with
+  // whole-wave stores (the outputs may lie in host memory, behind PCIe).
+  // s_sel holds them: its entries have moved to s_buf when the counting sort
+  // ranks them, and the rank sort reads s_buf.  Neither keeps more than
+  // kSelCap; the bitonic sort leaves them in place.
+  const uint64_t* sorted = s_sel;
+  auto emit = [&](uint32_t r, uint64_t c) { s_sel[r] = c; };
   if (sb == s_sel) {
     // Counting sort by bin, descending: an entry's position is the number of
     // selected entries in higher bins plus the number of larger keys in its
@@ -2323,9 +2325,32 @@ __global__ __launch_bounds__(kSelThreads) void k_select(SelectArgs a) {
     for (int i = (int)m + tid; i < n2; i += kSelThreads) sb[i] = 0ull;
     __syncthreads();
     bitonic_desc(sb, n2);
-    for (uint32_t i = tid; i < keep; i += kSelThreads) emit(i, sb[i]);
+    sorted = sb;
   }
   __syncthreads();
+  for (uint32_t i = tid; i < K; i += kSelThreads) {
+    const uint64_t c = i < keep ? sorted[i] : 0ull;
+    const uint32_t row = ~(uint32_t)c;
+    a.out_ids[(uint64_t)q * K + i] = i < keep ? ((uint64_t)(row >> 6) << 16) | (uint64_t)(row & 63u) : 0ull;
+    a.out_scores[(uint64_t)q * K + i] = i < keep ? key_score((uint32_t)(c >> 32)) : 0.0f;
+  }
+  if (a.stats_sum && q == 0) {
+    // every counter is final but this launch's own: 512 threads hold one each
+    // (counter t % 8 of copy t / 8), lanes of equal counter add up first
+    static_assert(kStatCopies == 64 && kStatCount == 8, "512 counters, eight of a kind per wave");
+    unsigned long long* s_sum = reinterpret_cast<unsigned long long*>(s_buf);
+    __syncthreads();  // s_buf is read no more
+    if (tid < 8) s_sum[tid] = 0ull;
+    __syncthreads();
+    if (tid < kStatCopies * kStatCount) {
+      unsigned long long c = a.stats_src[tid];
+#pragma unroll
+      for (int o = 8; o < 64; o <<= 1) c += __shfl_xor(c, o);
+      if ((tid & 63) < 8) atomicAdd(&s_sum[tid & 7], c);
+    }
+    __syncthreads();
+    if (tid < 8) a.stats_sum[tid] = s_sum[tid];
+  }
   // leave this query's pass state clean for the next scan
   if (tid < (int)a.nseg) a.seg_count[(uint64_t)q * a.nseg + tid] = 0u;
   if (a.hist)

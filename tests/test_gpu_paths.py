@@ -324,3 +324,27 @@ def test_plan_codebooks_are_the_reference_literals(device):
     b1 = np.array([int(h, 16) for h in fx["B1"]["f32_bits"]], dtype=np.uint32)
     assert np.array_equal(np.ctypeslib.as_array(p.eden_codebook).astype(np.float32).view(np.uint32), b4)
     assert np.array_equal(np.ctypeslib.as_array(p.eden_mid_codebook).astype(np.float32).view(np.uint32), b1)
+
+
+@pytest.mark.parametrize("nq,n_rows,k", [(1, 64 * 300 + 5, 64), (3, 64 * 300, 2049), (9, 64 * 40 - 3, 4096),
+                                         (65, 64 * 300, 256), (1, 100, 256)])
+def test_synchronous_scan_equals_enqueued_scan(device, nq, n_rows, k):
+    """mrl_scan (selection into host memory, each of its sorts, lists shorter
+    than K) against mrl_scan_async + fetch: same lists, counts and counters."""
+    rng = np.random.default_rng(nq + k)
+    rows = normalized(rng, n_rows, 192)
+    ix = m.DeviceIndex.upload(m.encode_corpus(rows, 8), device)
+    plan = m.QueryPlan.from_query(normalized(rng, nq, 192), 192, device)
+    cfg = m.ScanConfig(shortlist_cand=k)
+    for _ in range(2):  # the counters accumulate on the device between calls
+        a = m.scan_batch(ix, plan, cfg)
+        res = m.DeviceResults(nq, k, device)
+        res.scan(ix, plan, cfg)
+        b = res.fetch()
+        assert np.array_equal(a.counts, b.counts) and np.all(a.counts == min(k, n_rows))
+        for q in range(nq):
+            n = int(a.counts[q])
+            assert np.array_equal(a.ids[q, :n], b.ids[q, :n])
+            assert np.array_equal(a.scores[q, :n].view(np.uint32), b.scores[q, :n].view(np.uint32))
+            assert not a.ids[q, n:].any() and not a.scores[q, n:].any()
+        assert a.stats == b.stats
