@@ -497,6 +497,16 @@ int mrl_encode_corpus_device_clustered(mrl_ctx *ctx, const float *d_matrix, uint
 /* Device memory on the context's GPU, for callers without a HIP allocator of
  * their own (no reference counterpart).  Copies are synchronous. */
 int mrl_device_alloc(mrl_ctx *ctx, size_t bytes, void **out);
+/* Pinned host memory for a caller's output arrays (no reference counterpart).
+ * Where out_ids and out_scores of mrl_scan / mrl_results_fetch (out_rows and
+ * out_scores of mrl_rerank_rows) lie in such blocks of the same context, the
+ * device writes them directly instead of through a staging copy; contents and
+ * results are the same either way.  A block keeps its context alive until it
+ * is freed; freed blocks are kept for the next mrl_host_alloc, at most 64 MiB
+ * of them.  MRL_ERR_OUT_OF_MEMORY once 512 MiB are in use on the context:
+ * ordinary memory serves then. */
+int mrl_host_alloc(mrl_ctx *ctx, size_t bytes, void **out);
+void mrl_host_free(mrl_ctx *ctx, void *p);
 void mrl_device_free(mrl_ctx *ctx, void *d_ptr);
 int mrl_copy_to_device(mrl_ctx *ctx, void *d_dst, const void *src, size_t bytes);
 int mrl_copy_to_host(mrl_ctx *ctx, void *dst, const void *d_src, size_t bytes);

@@ -62,6 +62,71 @@ struct ProfRecord {
   mrl_kernel_time info;
 };
 
+// Buffers kept between calls: a plan, a rerank or a ring merge takes one for
+// its lifetime and gives it back once the stream is done with it, instead of
+// allocating and freeing (above 1 MB a hipMalloc / hipFree pair costs 12-70 us,
+// and a free may wait for the device).  Sizes are powers of two; at most
+// kPoolKeep bytes stay in a pool, all of them are freed with the context, and
+// an allocation that fails frees them first.  Own mutex: plans are destroyed
+// without the context lock.
+static const size_t kPoolKeep = (size_t)64 << 20;
+struct BlockPool {
+  explicit BlockPool(bool pinned_) : pinned(pinned_) {}
+  const bool pinned;
+  std::mutex mu;
+  std::vector<std::pair<uint8_t*, size_t>> free_blocks;
+  size_t kept = 0;
+  static size_t rounded(size_t bytes) {
+    size_t r = 4096;
+    while (r < bytes) r <<= 1;
+    return r;
+  }
+  void release(uint8_t* p) const { (void)(pinned ? hipHostFree(p) : hipFree(p)); }
+  // null: out of memory
+  uint8_t* take(size_t bytes) {
+    bytes = rounded(bytes);
+    {
+      std::lock_guard<std::mutex> g(mu);
+      for (size_t i = 0; i < free_blocks.size(); ++i)
+        if (free_blocks[i].second == bytes) {
+          uint8_t* p = free_blocks[i].first;
+          free_blocks[i] = free_blocks.back();
+          free_blocks.pop_back();
+          kept -= bytes;
+          return p;
+        }
+    }
+    for (int attempt = 0; attempt < 2; ++attempt) {
+      void* p = nullptr;
+      if ((pinned ? hipHostMalloc(&p, bytes, hipHostMallocDefault) : hipMalloc(&p, bytes)) == hipSuccess)
+        return static_cast<uint8_t*>(p);
+      (void)hipGetLastError();  // do not leave the failure for the next launch check
+      trim();
+    }
+    return nullptr;
+  }
+  // The device no longer uses p (taken with this size).
+  void give(void* p, size_t bytes) {
+    if (!p) return;
+    bytes = rounded(bytes);
+    {
+      std::lock_guard<std::mutex> g(mu);
+      if (kept + bytes <= kPoolKeep) {
+        free_blocks.emplace_back(static_cast<uint8_t*>(p), bytes);
+        kept += bytes;
+        return;
+      }
+    }
+    release(static_cast<uint8_t*>(p));
+  }
+  void trim() {
+    std::lock_guard<std::mutex> g(mu);
+    for (auto& b : free_blocks) release(b.first);
+    free_blocks.clear();
+    kept = 0;
+  }
+};
+
 struct mrl_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -78,6 +143,11 @@ struct mrl_ctx {
   uint32_t crc_const = 0;
   void* h_stage = nullptr;            // pinned host staging for result read-back
   size_t h_stage_cap = 0;
+  BlockPool dev_pool{false};
+  BlockPool pin_pool{true};
+  std::mutex host_mu;
+  std::map<uintptr_t, size_t> host_blocks;  // live mrl_host_alloc blocks
+  size_t host_bytes = 0;
   mrl_results* spare = nullptr;       // result buffers kept between synchronous mrl_scan calls
   uint8_t* scratch = nullptr;         // this device's copy of `scratch` (mrl_scan_noalloc); null: lookup failed
   // per-scan scratch of the block selection (grown on demand): the cluster x
@@ -258,7 +328,10 @@ struct mrl_plans {
   uint64_t mid_seed = 0;
   float* d_queries = nullptr;  // owned copy, n_q * dims
   float* d_luts = nullptr;     // n_q * kQData scan constants written by the plan kernel
-  uint8_t* d_block = nullptr;  // one allocation holding all of the above
+  uint8_t* d_block = nullptr;  // one pool block holding all of the above
+  size_t d_bytes = 0;
+  uint8_t* h_in = nullptr;     // pinned pool block the host inputs are copied from
+  size_t h_bytes = 0;
   // The plans are built lazily: by the next call that reads them (flush_plans),
   // or inside a one-query sampling pass (k_scan's fused plan).
   mutable bool pending = false;
@@ -303,10 +376,14 @@ struct mrl_results {
   uint32_t* o_counts = nullptr;
   uint32_t* o_status = nullptr;
   unsigned long long* o_stats = nullptr;  // null unless mapped: counters summed over their copies
-  // Pinned memory of the mapped outputs (allocated by the first synchronous
-  // scan): status u32[n_q], counts u32[n_q], stats u64[kStatCount], then ids
-  // and scores as in the device block.
-  uint8_t* h_out = nullptr;
+  // Pinned pool blocks of the mapped outputs (taken by the first synchronous
+  // scan that needs them): status u32[n_q], counts u32[n_q], stats
+  // u64[kStatCount]; and ids u64[n_q][k], scores f32[n_q][k] of callers whose
+  // own arrays the device cannot write.
+  uint8_t* h_head = nullptr;
+  uint8_t* h_rows = nullptr;
+  size_t head_bytes() const { return (size_t)std::max<uint32_t>(n_q, 1) * 8 + kStatCount * 8; }
+  size_t rows_bytes() const { return (size_t)std::max<uint32_t>(n_q, 1) * k * 12; }
   void to_device_outputs() {
     o_ids = d_ids;
     o_scores = d_scores;
@@ -396,8 +473,53 @@ static void ctx_free(mrl_ctx* ctx) {
   }
   for (hipEvent_t e : ctx->event_pool) (void)hipEventDestroy(e);
   if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
+  ctx->dev_pool.trim();
+  ctx->pin_pool.trim();
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
+}
+
+// Pinned host memory for a caller's outputs, from the context's pool.
+static const size_t kHostBlocksMax = (size_t)512 << 20;
+extern "C" int mrl_host_alloc(mrl_ctx* ctx, size_t bytes, void** out) {
+  if (!ctx || !out || !bytes) return fail(MRL_ERR_INVALID_ARG, "null argument");
+  *out = nullptr;
+  const size_t r = BlockPool::rounded(bytes);
+  std::lock_guard<std::mutex> g(ctx->host_mu);
+  if (bytes > kHostBlocksMax || ctx->host_bytes + r > kHostBlocksMax)
+    return fail(MRL_ERR_OUT_OF_MEMORY, "mrl_host_alloc: the context's pinned blocks are in use");
+  HIP_TRY(hipSetDevice(ctx->device));
+  uint8_t* p = ctx->pin_pool.take(bytes);
+  if (!p) return fail(MRL_ERR_OUT_OF_MEMORY, "pinned host memory");
+  ctx->host_blocks[(uintptr_t)p] = r;
+  ctx->host_bytes += r;
+  ctx_retain(ctx);
+  *out = p;
+  return MRL_OK;
+}
+
+extern "C" void mrl_host_free(mrl_ctx* ctx, void* p) {
+  if (!ctx || !p) return;
+  {
+    std::lock_guard<std::mutex> g(ctx->host_mu);
+    auto it = ctx->host_blocks.find((uintptr_t)p);
+    if (it == ctx->host_blocks.end()) return;
+    const size_t r = it->second;
+    ctx->host_blocks.erase(it);
+    ctx->host_bytes -= r;
+    ctx->pin_pool.give(p, r);
+  }
+  ctx_release(ctx);
+}
+
+// Whether the device may write [p, p + bytes) directly: it lies in a live
+// mrl_host_alloc block of this context.
+static bool in_host_block(mrl_ctx* ctx, const void* p, size_t bytes) {
+  std::lock_guard<std::mutex> g(ctx->host_mu);
+  auto it = ctx->host_blocks.upper_bound((uintptr_t)p);
+  if (it == ctx->host_blocks.begin()) return false;
+  --it;
+  return (uintptr_t)p + bytes <= it->first + it->second;
 }
 
 extern "C" int mrl_ctx_synchronize(mrl_ctx* ctx) {
@@ -895,8 +1017,9 @@ static int plans_build_impl(mrl_ctx* ctx, const float* queries, bool on_device, 
   const size_t plan_bytes = sizeof(mrl_query_plan) * nq, lut_bytes = sizeof(float) * kQData * nq;
   const size_t qbytes = (size_t)n_q * dims * sizeof(float);
   const size_t in_bytes = (64 + 128) * sizeof(float) + qbytes;
-  if (hipMalloc(&p->d_block, plan_bytes + lut_bytes + in_bytes) != hipSuccess)
-    return fail(MRL_ERR_OUT_OF_MEMORY, "plans");
+  p->d_bytes = plan_bytes + lut_bytes + in_bytes;
+  p->d_block = ctx->dev_pool.take(p->d_bytes);
+  if (!p->d_block) return fail(MRL_ERR_OUT_OF_MEMORY, "plans");
   p->d_plans = reinterpret_cast<mrl_query_plan*>(p->d_block);
   p->d_luts = reinterpret_cast<float*>(p->d_block + plan_bytes);
   float* d_in = reinterpret_cast<float*>(p->d_block + plan_bytes + lut_bytes);
@@ -911,16 +1034,18 @@ static int plans_build_impl(mrl_ctx* ctx, const float* queries, bool on_device, 
   if (n_q) p->d_queries = d_in + 192;
   hipError_t e = hipSuccess;
   if (!on_device) {
-    uint8_t* h = host_stage(ctx, in_bytes);
-    if (!h) {
-      dev_free(p->d_block);
+    // (the plans keep their staging, so nothing waits for the copy)
+    p->h_bytes = in_bytes;
+    p->h_in = ctx->pin_pool.take(in_bytes);
+    if (!p->h_in) {
+      ctx->dev_pool.give(p->d_block, p->d_bytes);
       return fail(MRL_ERR_OUT_OF_MEMORY, "pinned staging buffer");
     }
-    float* hf = reinterpret_cast<float*>(h);
+    float* hf = reinterpret_cast<float*>(p->h_in);
     if (eden) memcpy(hf, eden->mean, 64 * sizeof(float));
     if (eden_mid) memcpy(hf + 64, eden_mid->mean, 128 * sizeof(float));
     if (n_q) memcpy(hf + 192, queries, qbytes);
-    e = hipMemcpyAsync(d_in, h, in_bytes, hipMemcpyHostToDevice, ctx->stream);
+    e = hipMemcpyAsync(d_in, hf, in_bytes, hipMemcpyHostToDevice, ctx->stream);
   } else {
     float means[192] = {0};
     if (eden) memcpy(means, eden->mean, 64 * sizeof(float));
@@ -929,18 +1054,12 @@ static int plans_build_impl(mrl_ctx* ctx, const float* queries, bool on_device, 
     if (e == hipSuccess && n_q) e = hipMemcpyAsync(d_in + 192, queries, qbytes, hipMemcpyDeviceToDevice, ctx->stream);
   }
   if (e != hipSuccess) {
-    dev_free(p->d_block);
+    (void)hipStreamSynchronize(ctx->stream);
+    ctx->dev_pool.give(p->d_block, p->d_bytes);
+    ctx->pin_pool.give(p->h_in, p->h_bytes);
     return fail(MRL_ERR_HIP, "plan inputs copy");
   }
-  int rc2 = MRL_OK;
   p->pending = true;  // built by the first call that reads the plans
-  // The pinned inputs are reused by the next call: wait for the copy (host path).
-  if (!rc2 && !on_device && hipStreamSynchronize(ctx->stream) != hipSuccess) rc2 = fail(MRL_ERR_HIP, "plan build");
-  if (rc2) {
-    (void)hipStreamSynchronize(ctx->stream);
-    dev_free(p->d_block);
-    return rc2;
-  }
   ctx_retain(ctx);
   *out = p.release();
   return MRL_OK;
@@ -991,7 +1110,8 @@ extern "C" void mrl_plans_destroy(mrl_plans* plans) {
   mrl_ctx* ctx = plans->ctx;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
-  dev_free(plans->d_block);
+  ctx->dev_pool.give(plans->d_block, plans->d_bytes);
+  ctx->pin_pool.give(plans->h_in, plans->h_bytes);
   delete plans;
   ctx_release(ctx);
 }
@@ -1023,7 +1143,8 @@ static ScanParams make_params(const mrl_scan_config* cfg, const mrl_time_range* 
 }
 
 static void results_free(mrl_results* r) {
-  if (r->h_out) (void)hipHostFree(r->h_out);
+  if (r->h_head) r->ctx->pin_pool.give(r->h_head, r->head_bytes());
+  if (r->h_rows) r->ctx->pin_pool.give(r->h_rows, r->rows_bytes());
   dev_free(r->d_out);
   dev_free(r->d_cand_score);
   dev_free(r->d_cand_row);
@@ -1890,9 +2011,24 @@ static int resolve_pending(mrl_ctx* ctx, mrl_results* res) {
 // One read-back of the results block into pinned memory: the head (status,
 // counts, stats) and the ids / scores rows of the first n_q queries.  Caller
 // holds the lock.
-static int read_back(mrl_ctx* ctx, mrl_results* res, uint32_t n_q, uint8_t** out) {
+// With ids and scores (arrays the device can write) the rows go there and
+// only the head to the staging buffer.
+static int read_back(mrl_ctx* ctx, mrl_results* res, uint32_t n_q, uint8_t** out, uint64_t* ids = nullptr,
+                     float* scores = nullptr) {
   const size_t nq = std::max<uint32_t>(res->n_q, 1), K = res->k;
   const size_t head = results_head_bytes((uint32_t)nq);
+  if (ids) {
+    uint8_t* h = host_stage(ctx, head);
+    if (!h) return fail(MRL_ERR_OUT_OF_MEMORY, "pinned staging buffer");
+    hipError_t e = hipMemcpyAsync(ids, res->d_ids, n_q * K * 8, hipMemcpyDeviceToHost, ctx->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(scores, res->d_scores, n_q * K * 4, hipMemcpyDeviceToHost, ctx->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(h, res->d_out, head, hipMemcpyDeviceToHost, ctx->stream);
+    const hipError_t es = hipStreamSynchronize(ctx->stream);  // also on an error: the arrays are the caller's
+    if (e != hipSuccess || es != hipSuccess)
+      return fail(MRL_ERR_HIP, std::string("results copy: ") + hipGetErrorString(e != hipSuccess ? e : es));
+    *out = h;
+    return MRL_OK;
+  }
   uint8_t* h = host_stage(ctx, res->out_bytes);
   if (!h) return fail(MRL_ERR_OUT_OF_MEMORY, "pinned staging buffer");
   if (n_q == nq) {
@@ -1947,15 +2083,19 @@ extern "C" int mrl_results_fetch(mrl_ctx* ctx, mrl_results* res, uint64_t* out_i
   HIP_TRY(hipSetDevice(ctx->device));
   const uint32_t n_q = res->last_plans ? res->last_plans->n_q : 0;
   uint8_t* h = nullptr;
-  int rc = read_back(ctx, res, n_q, &h);
+  const size_t nq = std::max<uint32_t>(res->n_q, 1), K = res->k;
+  const bool direct = out_ids && out_scores && n_q && in_host_block(ctx, out_ids, n_q * K * 8) &&
+                      in_host_block(ctx, out_scores, n_q * K * 4);
+  uint64_t* ids = direct ? out_ids : nullptr;
+  float* scores = direct ? out_scores : nullptr;
+  int rc = read_back(ctx, res, n_q, &h, ids, scores);
   if (rc) return rc;
   bool rerun = false;
   if ((rc = handle_scan_status(ctx, res, reinterpret_cast<const uint32_t*>(h), n_q, &rerun))) return rc;
-  if (rerun && (rc = read_back(ctx, res, n_q, &h))) return rc;
-  const size_t nq = std::max<uint32_t>(res->n_q, 1), K = res->k;
+  if (rerun && (rc = read_back(ctx, res, n_q, &h, ids, scores))) return rc;
   const size_t head = results_head_bytes((uint32_t)nq);
-  if (out_ids && n_q) memcpy(out_ids, h + head, n_q * K * 8);
-  if (out_scores && n_q) memcpy(out_scores, h + head + nq * K * 8, n_q * K * 4);
+  if (out_ids && n_q && !direct) memcpy(out_ids, h + head, n_q * K * 8);
+  if (out_scores && n_q && !direct) memcpy(out_scores, h + head + nq * K * 8, n_q * K * 4);
   if (out_counts && n_q) memcpy(out_counts, h + nq * 4, (size_t)n_q * 4);
   unsigned long long st[kStatCount] = {0};
   for (int c = 0; c < kStatCopies; ++c) {
@@ -2001,16 +2141,17 @@ static int scan_mapped(mrl_ctx* ctx, const mrl_index* index, const mrl_plans* pl
   HIP_TRY(hipSetDevice(ctx->device));
   const size_t nq = std::max<uint32_t>(res->n_q, 1);
   const uint32_t n_q = plans->n_q;
-  const size_t head = nq * 8 + kStatCount * 8;
-  if (!res->h_out && hipHostMalloc((void**)&res->h_out, head + nq * K * 12, hipHostMallocDefault) != hipSuccess) {
-    res->h_out = nullptr;
-    return fail(MRL_ERR_OUT_OF_MEMORY, "pinned result buffer");
-  }
-  res->o_status = reinterpret_cast<uint32_t*>(res->h_out);
+  // lists straight into the caller's arrays where the device can write them
+  const bool direct = out_ids && out_scores && n_q && in_host_block(ctx, out_ids, (size_t)n_q * K * 8) &&
+                      in_host_block(ctx, out_scores, (size_t)n_q * K * 4);
+  if (!res->h_head) res->h_head = ctx->pin_pool.take(res->head_bytes());
+  if (!direct && !res->h_rows) res->h_rows = ctx->pin_pool.take(res->rows_bytes());
+  if (!res->h_head || (!direct && !res->h_rows)) return fail(MRL_ERR_OUT_OF_MEMORY, "pinned result buffer");
+  res->o_status = reinterpret_cast<uint32_t*>(res->h_head);
   res->o_counts = res->o_status + nq;
-  res->o_stats = reinterpret_cast<unsigned long long*>(res->h_out + nq * 8);
-  res->o_ids = reinterpret_cast<uint64_t*>(res->h_out + head);
-  res->o_scores = reinterpret_cast<float*>(res->h_out + head + nq * K * 8);
+  res->o_stats = reinterpret_cast<unsigned long long*>(res->h_head + nq * 8);
+  res->o_ids = direct ? out_ids : reinterpret_cast<uint64_t*>(res->h_rows);
+  res->o_scores = direct ? out_scores : reinterpret_cast<float*>(res->h_rows + nq * K * 8);
   bool sampled, rerun;
   rc = enqueue_scan_into(ctx, index, plans, cfg, time, res, K, &sampled);
   if (!rc && hipStreamSynchronize(ctx->stream) != hipSuccess) rc = fail(MRL_ERR_HIP, "scan");
@@ -2040,8 +2181,8 @@ static int scan_mapped(mrl_ctx* ctx, const mrl_index* index, const mrl_plans* pl
     res->pending = false;
   }
   if (!rc) {
-    if (out_ids && n_q) memcpy(out_ids, res->o_ids, (size_t)n_q * K * 8);
-    if (out_scores && n_q) memcpy(out_scores, res->o_scores, (size_t)n_q * K * 4);
+    if (out_ids && n_q && !direct) memcpy(out_ids, res->o_ids, (size_t)n_q * K * 8);
+    if (out_scores && n_q && !direct) memcpy(out_scores, res->o_scores, (size_t)n_q * K * 4);
     if (out_counts && n_q) memcpy(out_counts, res->o_counts, (size_t)n_q * 4);
     take_stats(res, st, stats);
   }
@@ -2721,38 +2862,56 @@ extern "C" int mrl_rerank_rows(mrl_ctx* ctx, const mrl_rerank_store* store, cons
   if (stride > MRL_MAX_SHORTLIST) return fail(MRL_ERR_INVALID_ARG, "stride above MRL_MAX_SHORTLIST");
   if (n_q == 0 || stride == 0) return MRL_OK;
   if (!queries || !cand_rows || !counts || !out_rows || !out_scores) return fail(MRL_ERR_INVALID_ARG, "null buffer");
-  for (uint32_t q = 0; q < n_q; ++q) {
+  for (uint32_t q = 0; q < n_q; ++q)
     if (counts[q] > stride) return fail(MRL_ERR_INVALID_ARG, "count above stride");
-    for (uint32_t i = 0; i < counts[q]; ++i)
-      if (cand_rows[(size_t)q * stride + i] >= store->n_rows)
-        return fail(MRL_ERR_INVALID_ARG, "candidate row out of range of the rerank store");
-  }
   std::lock_guard<std::mutex> g(ctx->mu);
   HIP_TRY(hipSetDevice(ctx->device));
+  // One pool block on each side, laid out alike but for the device's scratch:
+  // the outputs (status, counts, rows, scores: one copy back), then the inputs
+  // [candidates][queries][counts] (one copy in).
   const size_t nc = (size_t)n_q * stride;
   const size_t qbytes = (size_t)n_q * dims * 4;
-  const size_t bytes = rerank_bytes(n_q, stride) + qbytes + nc * 8 + (size_t)n_q * 4 + 64;
-  uint8_t* base = nullptr;
-  if (hipMalloc(&base, bytes) != hipSuccess) return fail(MRL_ERR_OUT_OF_MEMORY, "rerank buffers");
-  const RerankBuffers b = rerank_carve(base, n_q, stride);
-  uint8_t* p = base + ((rerank_bytes(n_q, stride) + 15) & ~(size_t)15);
-  uint64_t* d_cand = reinterpret_cast<uint64_t*>(p);
-  float* d_q = reinterpret_cast<float*>(p + nc * 8);
-  uint32_t* d_counts = reinterpret_cast<uint32_t*>(p + nc * 8 + qbytes);
-  hipError_t e = hipMemcpyAsync(d_cand, cand_rows, nc * 8, hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(d_q, queries, qbytes, hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(d_counts, counts, (size_t)n_q * 4, hipMemcpyHostToDevice, ctx->stream);
-  int rc = MRL_OK;
-  if (e == hipSuccess) rc = enqueue_rerank(ctx, store, d_q, n_q, d_cand, 0, d_counts, stride, b);
-  std::vector<uint32_t> st(n_q);
-  if (e == hipSuccess && !rc) e = hipMemcpyAsync(out_rows, b.out_rows, nc * 8, hipMemcpyDeviceToHost, ctx->stream);
-  if (e == hipSuccess && !rc) e = hipMemcpyAsync(out_scores, b.out_scores, nc * 4, hipMemcpyDeviceToHost, ctx->stream);
-  if (e == hipSuccess && !rc) e = hipMemcpyAsync(st.data(), b.status, (size_t)n_q * 4, hipMemcpyDeviceToHost, ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  dev_free(base);
-  if (rc) return rc;
-  if (e != hipSuccess) return fail(MRL_ERR_HIP, std::string("rerank: ") + hipGetErrorString(e));
-  return status_error(st.data(), (uint32_t)st.size());
+  const size_t in_at = (rerank_bytes(n_q, stride) + 15) & ~(size_t)15;
+  const size_t in_bytes = nc * 8 + qbytes + (size_t)n_q * 4;
+  const size_t out_bytes = (rerank_out_bytes(n_q, stride) + 15) & ~(size_t)15;
+  uint8_t* base = ctx->dev_pool.take(in_at + in_bytes);
+  uint8_t* h = base ? ctx->pin_pool.take(out_bytes + in_bytes) : nullptr;
+  int rc = h ? MRL_OK : fail(MRL_ERR_OUT_OF_MEMORY, "rerank buffers");
+  if (!rc) {
+    // (the kernels check every used row against the store: status bit 1)
+    memcpy(h + out_bytes, cand_rows, nc * 8);
+    memcpy(h + out_bytes + nc * 8, queries, qbytes);
+    memcpy(h + out_bytes + nc * 8 + qbytes, counts, (size_t)n_q * 4);
+  }
+  if (!rc) {
+    const RerankBuffers b = rerank_carve(base, n_q, stride);
+    uint64_t* d_cand = reinterpret_cast<uint64_t*>(base + in_at);
+    float* d_q = reinterpret_cast<float*>(base + in_at + nc * 8);
+    uint32_t* d_counts = reinterpret_cast<uint32_t*>(base + in_at + nc * 8 + qbytes);
+    hipError_t e = hipMemcpyAsync(d_cand, h + out_bytes, in_bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) rc = enqueue_rerank(ctx, store, d_q, n_q, d_cand, 0, d_counts, stride, b);
+    const bool direct = in_host_block(ctx, out_rows, nc * 8) && in_host_block(ctx, out_scores, nc * 4);
+    if (e == hipSuccess && !rc) {
+      if (direct) {
+        e = hipMemcpyAsync(out_rows, b.out_rows, nc * 8, hipMemcpyDeviceToHost, ctx->stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(out_scores, b.out_scores, nc * 4, hipMemcpyDeviceToHost, ctx->stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(h, b.status, (size_t)n_q * 8, hipMemcpyDeviceToHost, ctx->stream);
+      } else {
+        e = hipMemcpyAsync(h, b.status, rerank_out_bytes(n_q, stride), hipMemcpyDeviceToHost, ctx->stream);
+      }
+    }
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = es;
+    if (!rc && e != hipSuccess) rc = fail(MRL_ERR_HIP, std::string("rerank: ") + hipGetErrorString(e));
+    if (!rc && !direct) {
+      memcpy(out_rows, h + (size_t)n_q * 8, nc * 8);
+      memcpy(out_scores, h + (size_t)n_q * 8 + nc * 8, nc * 4);
+    }
+    if (!rc) rc = status_error(reinterpret_cast<const uint32_t*>(h), n_q);
+  }
+  if (base) ctx->dev_pool.give(base, in_at + in_bytes);
+  if (h) ctx->pin_pool.give(h, out_bytes + in_bytes);
+  return rc;
 }
 
 extern "C" int mrl_results_rerank(mrl_ctx* ctx, mrl_results* res, const mrl_rerank_store* store, uint64_t* out_rows,

@@ -10,6 +10,8 @@ from __future__ import annotations
 import ctypes as C
 import os
 
+import numpy as np
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), "_build", "libmrl_scan.so")
 
@@ -154,6 +156,10 @@ _F = C.POINTER(C.c_float)
 _U32 = C.POINTER(C.c_uint32)
 _U64 = C.POINTER(C.c_uint64)
 
+# an array's address as a plain integer (`addr`): the entry points called once
+# per query batch take their arrays this way, a pointer object costs 1 us each
+_A = C.c_void_p
+
 # name -> (restype, argtypes); every symbol declared in include/*.h
 SIGNATURES = {
     "mrl_abi_version": (C.c_int, []),
@@ -167,7 +173,7 @@ SIGNATURES = {
     "mrl_index_block_count": (C.c_int, [_P, _U64]),
     "mrl_index_download": (C.c_int, [_P, _P, _P]),
     "mrl_index_destroy": (None, [_P]),
-    "mrl_plans_build": (C.c_int, [_P, _F, C.c_uint32, C.c_uint32, C.c_int, C.c_int,
+    "mrl_plans_build": (C.c_int, [_P, _A, C.c_uint32, C.c_uint32, C.c_int, C.c_int,
                                    C.POINTER(EdenFitC), C.POINTER(EdenFitC), _PP]),
     "mrl_plans_build_device": (C.c_int, [_P, _P, C.c_uint32, C.c_uint32, C.c_int, C.c_int,
                                           C.POINTER(EdenFitC), C.POINTER(EdenFitC), _PP]),
@@ -175,12 +181,12 @@ SIGNATURES = {
     "mrl_plans_count": (C.c_int, [_P, _U32]),
     "mrl_plans_export": (C.c_int, [_P, _P, C.c_uint32, C.c_uint32, C.POINTER(QueryPlanC)]),
     "mrl_plans_destroy": (None, [_P]),
-    "mrl_scan": (C.c_int, [_P, _P, _P, C.POINTER(ScanConfigC), C.POINTER(TimeRangeC), _U64, _F, _U32,
+    "mrl_scan": (C.c_int, [_P, _P, _P, C.POINTER(ScanConfigC), C.POINTER(TimeRangeC), _A, _A, _A,
                            C.POINTER(ScanStatsC)]),
     "mrl_results_create": (C.c_int, [_P, C.c_uint32, C.c_uint32, _PP]),
     "mrl_results_destroy": (None, [_P]),
     "mrl_scan_async": (C.c_int, [_P, _P, _P, C.POINTER(ScanConfigC), C.POINTER(TimeRangeC), _P]),
-    "mrl_results_fetch": (C.c_int, [_P, _P, _U64, _F, _U32, C.POINTER(ScanStatsC)]),
+    "mrl_results_fetch": (C.c_int, [_P, _P, _A, _A, _A, C.POINTER(ScanStatsC)]),
     "mrl_results_floors": (C.c_int, [_P, _P, _F]),
     "mrl_scan_noalloc": (C.c_int, [_P, _P, _P, C.POINTER(ScanConfigC), C.POINTER(TimeRangeC), _P, _P, _P, _P]),
     "mrl_scan_fixed_tau": (C.c_int, [_P, _P, _P, C.POINTER(ScanConfigC), C.POINTER(TimeRangeC), _F, _U64,
@@ -203,6 +209,8 @@ SIGNATURES = {
     "mrl_encode_corpus_device_clustered": (C.c_int, [_P, _P, C.c_uint64, C.c_uint32, _P, C.c_uint32,
                                                      C.POINTER(EdenFitC), C.POINTER(EdenFitC), _P]),
     "mrl_index_from_device": (C.c_int, [_P, _P, C.c_uint64, _PP]),
+    "mrl_host_alloc": (C.c_int, [_P, C.c_size_t, _PP]),
+    "mrl_host_free": (None, [_P, _P]),
     "mrl_device_alloc": (C.c_int, [_P, C.c_size_t, _PP]),
     "mrl_device_free": (None, [_P, _P]),
     "mrl_device_mem_info": (C.c_int, [_P, _U64, _U64]),
@@ -211,10 +219,10 @@ SIGNATURES = {
     "mrl_rerank_store_create": (C.c_int, [_P, _P, C.c_int, C.c_uint64, C.c_uint32, C.c_int, _PP]),
     "mrl_rerank_store_destroy": (None, [_P]),
     "mrl_rerank_store_download": (C.c_int, [_P, _P, _P, C.POINTER(C.c_uint16)]),
-    "mrl_rerank_rows": (C.c_int, [_P, _P, _F, C.c_uint32, C.c_uint32, _U64, _U32, C.c_uint32, _U64, _F]),
-    "mrl_results_rerank": (C.c_int, [_P, _P, _P, _U64, _F, _U32]),
-    "mrl_ring_search": (C.c_int, [_P, _F, C.c_uint32, C.c_uint32, _F, C.c_uint32, C.c_uint32, _U64, _F, _U32]),
-    "mrl_results_merge_ring": (C.c_int, [_P, _P, _F, C.c_uint32, C.c_uint32]),
+    "mrl_rerank_rows": (C.c_int, [_P, _P, _A, C.c_uint32, C.c_uint32, _A, _A, C.c_uint32, _A, _A]),
+    "mrl_results_rerank": (C.c_int, [_P, _P, _P, _A, _A, _A]),
+    "mrl_ring_search": (C.c_int, [_P, _A, C.c_uint32, C.c_uint32, _A, C.c_uint32, C.c_uint32, _A, _A, _A]),
+    "mrl_results_merge_ring": (C.c_int, [_P, _P, _A, C.c_uint32, C.c_uint32]),
     "mrl_synth_docs": (C.c_int, [C.POINTER(SynthSpecC), C.c_uint64, C.c_uint64, C.c_int, _F]),
     "mrl_synth_queries": (C.c_int, [C.POINTER(SynthSpecC), C.c_uint64, C.c_float, C.c_int, C.c_uint32, _F,
                                     _U64]),
@@ -248,6 +256,11 @@ def check(rc: int) -> None:
         raise MrlError(rc, msg.decode() if msg else "")
 
 
+def addr(a) -> int:
+    """Address of an array's data."""
+    return a.__array_interface__["data"][0]
+
+
 def fptr(a):
     """float* view of a contiguous float32 numpy array."""
     return a.ctypes.data_as(_F)
@@ -259,6 +272,50 @@ def u32ptr(a):
 
 def u64ptr(a):
     return a.ctypes.data_as(_U64)
+
+
+# Output arrays of at least this many bytes are placed in pinned memory, where
+# the device writes them directly: below, a copy out of the library's staging
+# buffer costs less than the array's bookkeeping.
+PINNED_MIN_BYTES = 1 << 17
+
+
+class _HostBlock:
+    """A mrl_host_alloc block; numpy arrays made from it keep it alive."""
+
+    __slots__ = ("_free", "_ctx", "_ptr", "__array_interface__")
+
+    def __init__(self, ctx, nbytes: int):
+        p = C.c_void_p()
+        self._ptr = None
+        self._free = lib.mrl_host_free
+        check(lib.mrl_host_alloc(ctx, nbytes, C.byref(p)))
+        # the block keeps the context alive, whatever becomes of the Device object
+        self._ctx, self._ptr = C.c_void_p(ctx.value), p
+        self.__array_interface__ = {"shape": (nbytes,), "typestr": "|u1", "data": (p.value, False), "version": 3}
+
+    def __del__(self):
+        if self._ptr:
+            self._free(self._ctx, self._ptr)
+            self._ptr = None
+
+
+def lists(ctx, n_q: int, k: int):
+    """Output arrays of n_q lists of k: (uint64 (n_q, k), float32 (n_q, k),
+    their two addresses), pinned when large (zeroed ordinary memory otherwise,
+    or when the context has no pinned memory left)."""
+    n = n_q * k
+    raw = None
+    if n * 12 >= PINNED_MIN_BYTES:
+        try:
+            raw = np.asarray(_HostBlock(ctx, n * 12))
+        except MrlError as e:
+            if e.code != MRL_ERR_OUT_OF_MEMORY:
+                raise
+    if raw is None:
+        raw = np.zeros(n * 12, dtype=np.uint8)
+    at = addr(raw)
+    return (np.ndarray((n_q, k), np.uint64, raw), np.ndarray((n_q, k), np.float32, raw, n * 8), at, at + n * 8)
 
 
 def vptr(a):

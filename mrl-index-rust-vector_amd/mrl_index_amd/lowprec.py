@@ -120,11 +120,9 @@ def rerank_batch(store: RerankStore, queries, cand_rows, counts=None) -> Tuple[n
     if q.shape != (n_q, store.dims):
         raise ValueError("queries must be (n_q, dims) with one row per candidate list")
     cnt = np.full(n_q, stride, dtype=np.uint32) if counts is None else np.ascontiguousarray(counts, dtype=np.uint32)
-    rows = np.zeros((n_q, stride), dtype=np.uint64)
-    scores = np.zeros((n_q, stride), dtype=np.float32)
-    _lib.check(_lib.lib.mrl_rerank_rows(store.device.handle, store.handle, _lib.fptr(q), n_q, store.dims,
-                                        _lib.u64ptr(c), _lib.u32ptr(cnt), stride, _lib.u64ptr(rows),
-                                        _lib.fptr(scores)))
+    rows, scores, at_rows, at_scores = _lib.lists(store.device.handle, n_q, stride)
+    _lib.check(_lib.lib.mrl_rerank_rows(store.device.handle, store.handle, _lib.addr(q), n_q, store.dims,
+                                        _lib.addr(c), _lib.addr(cnt), stride, at_rows, at_scores))
     return rows, scores
 
 

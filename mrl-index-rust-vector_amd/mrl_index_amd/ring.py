@@ -91,8 +91,8 @@ class RingBuffer:
         sc = np.zeros((1, max(keep, 1)), dtype=np.float32)
         cnt = np.zeros(1, dtype=np.uint32)
         dev = self.device or default_device()
-        _lib.check(_lib.lib.mrl_ring_search(dev.handle, _lib.fptr(rows), rows.shape[0], rows.shape[1], _lib.fptr(q),
-                                            1, top_k, _lib.u64ptr(loc), _lib.fptr(sc), _lib.u32ptr(cnt)))
+        _lib.check(_lib.lib.mrl_ring_search(dev.handle, _lib.addr(rows), rows.shape[0], rows.shape[1], _lib.addr(q),
+                                            1, top_k, _lib.addr(loc), _lib.addr(sc), _lib.addr(cnt)))
         return [(int(loc[0, i]), float(sc[0, i]), self.pending[int(loc[0, i])]) for i in range(int(cnt[0]))]
 
     def merge_into(self, results: DeviceResults) -> None:
@@ -100,5 +100,5 @@ class RingBuffer:
         if not self.pending:
             return
         rows = self.pending_matrix()
-        _lib.check(_lib.lib.mrl_results_merge_ring(results.device.handle, results._h, _lib.fptr(rows),
+        _lib.check(_lib.lib.mrl_results_merge_ring(results.device.handle, results._h, _lib.addr(rows),
                                                    rows.shape[0], rows.shape[1]))

@@ -197,7 +197,7 @@ class QueryPlan:
         h = C.c_void_p()
         ef = eden.to_c() if eden is not None else None
         mf = eden_mid.to_c() if eden_mid is not None else None
-        _lib.check(_lib.lib.mrl_plans_build(device.handle, _lib.fptr(q), q.shape[0], dims, int(prefix_codec),
+        _lib.check(_lib.lib.mrl_plans_build(device.handle, _lib.addr(q), q.shape[0], dims, int(prefix_codec),
                                             int(mid_codec), C.byref(ef) if ef else None,
                                             C.byref(mf) if mf else None, C.byref(h)))
         return cls(h, device, q.shape[0], dims, prefix_codec, mid_codec, (eden, eden_mid))
@@ -310,14 +310,13 @@ def scan_batch(blocks: Union["DeviceIndex", np.ndarray], plan: QueryPlan, cfg, t
     try:
         k = max(int(sc.shortlist_cand), 1)
         nq = plan.n_queries
-        ids = np.zeros((nq, k), dtype=np.uint64)
-        scores = np.zeros((nq, k), dtype=np.float32)
+        ids, scores, at_ids, at_scores = _lib.lists(plan.device.handle, nq, k)
         counts = np.zeros(nq, dtype=np.uint32)
         st = _lib.ScanStatsC()
         c = sc.to_c()
         t = _time(time_lo, time_hi)
         _lib.check(_lib.lib.mrl_scan(plan.device.handle, idx.handle, plan.handle, C.byref(c), C.byref(t),
-                                     _lib.u64ptr(ids), _lib.fptr(scores), _lib.u32ptr(counts), C.byref(st)))
+                                     at_ids, at_scores, _lib.addr(counts), C.byref(st)))
         return ScanResult(ids, scores, counts, ScanStats.from_c(st))
     finally:
         if owned:
@@ -367,12 +366,11 @@ class DeviceResults:
 
     def fetch(self) -> ScanResult:
         nq, k = self._nq, self.k
-        ids = np.zeros((nq, k), dtype=np.uint64)
-        scores = np.zeros((nq, k), dtype=np.float32)
+        ids, scores, at_ids, at_scores = _lib.lists(self.device.handle, nq, k)
         counts = np.zeros(nq, dtype=np.uint32)
         st = _lib.ScanStatsC()
-        _lib.check(_lib.lib.mrl_results_fetch(self.device.handle, self._h, _lib.u64ptr(ids), _lib.fptr(scores),
-                                              _lib.u32ptr(counts), C.byref(st)))
+        _lib.check(_lib.lib.mrl_results_fetch(self.device.handle, self._h, at_ids, at_scores, _lib.addr(counts),
+                                              C.byref(st)))
         return ScanResult(ids, scores, counts, ScanStats.from_c(st))
 
     def floors(self) -> np.ndarray:
@@ -387,11 +385,10 @@ class DeviceResults:
         every query's shortlist against ``store`` (a RerankStore): returns
         (rows (n_q, K), scores (n_q, K), counts (n_q,))."""
         nq, k = self._nq, self.k
-        rows = np.zeros((nq, k), dtype=np.uint64)
-        scores = np.zeros((nq, k), dtype=np.float32)
+        rows, scores, at_rows, at_scores = _lib.lists(self.device.handle, nq, k)
         counts = np.zeros(nq, dtype=np.uint32)
-        _lib.check(_lib.lib.mrl_results_rerank(self.device.handle, self._h, store.handle, _lib.u64ptr(rows),
-                                               _lib.fptr(scores), _lib.u32ptr(counts)))
+        _lib.check(_lib.lib.mrl_results_rerank(self.device.handle, self._h, store.handle, at_rows, at_scores,
+                                               _lib.addr(counts)))
         return rows, scores, counts
 
     def close(self):

@@ -2,6 +2,7 @@
 alive, so the context and its objects may be destroyed in any order
 (include/mrl_scan.h), and a process that exits with handles still open exits
 normally."""
+import ctypes as C
 import itertools
 import os
 import subprocess
@@ -102,3 +103,48 @@ def test_process_exit_with_open_handles(device, small):
     p = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=110)
     assert p.returncode == 0, p.stderr[-2000:]
     assert "done" in p.stdout and "terminate" not in p.stderr
+
+
+def test_large_result_arrays_outlive_their_context():
+    """Large result lists are pinned blocks of the context the device writes
+    directly: equal to the lists of small calls, intact after the device, index
+    and plans are gone, ordinary memory once the context's pinned blocks are in
+    use, and blocks are reused once their arrays are."""
+    rng = np.random.default_rng(8)
+    rows = normalized(rng, 64 * 300, 192)
+    qs = normalized(rng, 48, 192)
+    dev = m.Device(0)
+    ix = m.DeviceIndex.upload(m.encode_corpus(rows, 8), dev)
+    cfg = m.ScanConfig(shortlist_cand=256)
+    plan = m.QueryPlan.from_query(qs, 192, dev)
+    big = m.scan_batch(ix, plan, cfg)
+    assert big.ids.nbytes + big.scores.nbytes >= m._lib.PINNED_MIN_BYTES
+    res = m.DeviceResults(48, 256, dev)
+    res.scan(ix, plan, cfg)
+    fetched = res.fetch()
+    small = [m.scan_batch(ix, m.QueryPlan.from_query(qs[i:i + 24], 192, dev), cfg) for i in (0, 24)]
+    assert small[0].ids.nbytes + small[0].scores.nbytes < m._lib.PINNED_MIN_BYTES
+    want_ids = np.concatenate([r.ids for r in small])
+    want = np.concatenate([r.scores for r in small]).view(np.uint32)
+    hold, p = [], C.c_void_p()
+    for size in (64 << 20, 1 << 20, 1 << 18):
+        while L.mrl_host_alloc(dev.handle, size, C.byref(p)) == 0:
+            hold.append(C.c_void_p(p.value))
+    full = m.scan_batch(ix, plan, cfg)  # no pinned memory left
+    handle = C.c_void_p(dev.handle.value)
+    for h in hold:
+        L.mrl_host_free(handle, h)
+    for o in (res, plan, ix, dev):
+        o.close()
+    for r in (big, fetched, full):
+        assert np.array_equal(r.ids, want_ids) and np.array_equal(r.scores.view(np.uint32), want)
+    # a freed block serves the next call
+    dev = m.Device(0)
+    ix = m.DeviceIndex.upload(m.encode_corpus(rows, 8), dev)
+    plan = m.QueryPlan.from_query(qs, 192, dev)
+    a = m.scan_batch(ix, plan, cfg)
+    at = a.ids.ctypes.data
+    del a
+    assert m.scan_batch(ix, plan, cfg).ids.ctypes.data == at
+    for o in (plan, ix, dev):
+        o.close()
