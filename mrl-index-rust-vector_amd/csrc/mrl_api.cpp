@@ -2986,6 +2986,30 @@ static int check_ring_args(const float* pending, uint32_t n_pending, uint32_t di
   return MRL_OK;
 }
 
+// The fused ring kernel's call: the pending rows (and, for a search, the
+// queries) go to a pool block with one copy; `run` enqueues the launches and
+// waits.  Caller holds the lock.  h: pinned, [inputs][out_bytes of outputs].
+struct RingBlocks {
+  mrl_ctx* ctx;
+  size_t in_bytes, out_bytes;
+  uint8_t *d = nullptr, *h = nullptr;
+  RingBlocks(mrl_ctx* c, size_t in, size_t out) : ctx(c), in_bytes((in + 15) & ~(size_t)15), out_bytes(out) {
+    d = ctx->dev_pool.take(in_bytes);
+    h = d ? ctx->pin_pool.take(in_bytes + out_bytes) : nullptr;
+  }
+  uint8_t* out() const { return h + in_bytes; }
+  ~RingBlocks() {
+    (void)hipStreamSynchronize(ctx->stream);
+    if (d) ctx->dev_pool.give(d, in_bytes);
+    if (h) ctx->pin_pool.give(h, in_bytes + out_bytes);
+  }
+};
+static int ring_status_error(const uint32_t* st, uint32_t n) {
+  for (uint32_t q = 0; q < n; ++q)
+    if (st[q] & 0x100u) return fail(MRL_ERR_NAN, "NaN rerank score (partial_cmp().unwrap() would panic)");
+  return MRL_OK;
+}
+
 extern "C" int mrl_ring_search(mrl_ctx* ctx, const float* pending, uint32_t n_pending, uint32_t dims,
                                const float* queries, uint32_t n_q, uint32_t top_k, uint64_t* out_local,
                                float* out_scores, uint32_t* out_counts) {
@@ -3002,6 +3026,31 @@ extern "C" int mrl_ring_search(mrl_ctx* ctx, const float* pending, uint32_t n_pe
   }
   std::lock_guard<std::mutex> g(ctx->mu);
   HIP_TRY(hipSetDevice(ctx->device));
+  const size_t pbytes = (size_t)n_pending * dims * 4;
+  if (n_pending <= kRingFused) {
+    const size_t nk = (size_t)n_q * keep;
+    RingBlocks rb(ctx, pbytes + (size_t)n_q * dims * 4, nk * 12 + (size_t)n_q * 4);
+    if (!rb.h) return fail(MRL_ERR_OUT_OF_MEMORY, "ring search buffers");
+    memcpy(rb.h, pending, pbytes);
+    memcpy(rb.h + pbytes, queries, (size_t)n_q * dims * 4);
+    HIP_TRY(hipMemcpyAsync(rb.d, rb.h, pbytes + (size_t)n_q * dims * 4, hipMemcpyHostToDevice, ctx->stream));
+    RingArgs ra{};
+    ra.rows = reinterpret_cast<const float*>(rb.d);
+    ra.queries = reinterpret_cast<const float*>(rb.d + pbytes);
+    ra.n_ring = n_pending;
+    ra.dims = dims;
+    ra.n_q = n_q;
+    ra.keep = keep;
+    ra.out_local = reinterpret_cast<uint64_t*>(rb.out());
+    ra.out_scores = reinterpret_cast<float*>(rb.out() + nk * 8);
+    ra.out_status = reinterpret_cast<uint32_t*>(rb.out() + nk * 12);
+    HIP_TRY(launch_ring(ra, ctx->stream));
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    memcpy(out_local, ra.out_local, nk * 8);
+    memcpy(out_scores, ra.out_scores, nk * 4);
+    for (uint32_t q = 0; q < n_q; ++q) out_counts[q] = keep;
+    return ring_status_error(ra.out_status, n_q);
+  }
   float* d_q = nullptr;
   mrl_rerank_store* store = nullptr;
   void* scratch = nullptr;
@@ -3042,9 +3091,49 @@ extern "C" int mrl_results_merge_ring(mrl_ctx* ctx, mrl_results* res, const floa
   const mrl_plans* plans = res->last_plans;
   if (!plans) return fail(MRL_ERR_INVALID_ARG, "no scan was enqueued on these results");
   if (plans->dims != dims) return fail(MRL_ERR_INVALID_ARG, "pending rows have other dims than the queries");
-  if ((rc = resolve_pending(ctx, res))) return rc;
   const uint32_t n_q = plans->n_q, K = res->k;
-  if (n_q == 0 || n_pending == 0) return MRL_OK;
+  if (n_q == 0 || n_pending == 0 || !res->last_index || !res->last_index->n_blocks || n_pending > kRingFused) {
+    if ((rc = resolve_pending(ctx, res))) return rc;
+    if (n_q == 0 || n_pending == 0) return MRL_OK;
+  }
+  if (n_pending <= kRingFused) {
+    // Enqueued behind the scan: the launch merges unless a query of the scan
+    // needs the host (a NaN, an overflowed list), which resolves the scan
+    // and launches again.
+    const size_t pbytes = (size_t)n_pending * dims * 4;
+    RingBlocks rb(ctx, pbytes, (size_t)n_q * 4);
+    if (!rb.h) return fail(MRL_ERR_OUT_OF_MEMORY, "ring merge");
+    memcpy(rb.h, pending, pbytes);
+    HIP_TRY(hipMemcpyAsync(rb.d, rb.h, pbytes, hipMemcpyHostToDevice, ctx->stream));
+    RingArgs ra{};
+    ra.rows = reinterpret_cast<const float*>(rb.d);
+    ra.queries = plans->d_queries;
+    ra.n_ring = n_pending;
+    ra.dims = dims;
+    ra.n_q = n_q;
+    ra.k = K;
+    ra.ids = res->d_ids;
+    ra.scores = res->d_scores;
+    ra.counts = res->d_counts;
+    ra.gate = res->pending ? res->d_status : nullptr;
+    ra.out_status = reinterpret_cast<uint32_t*>(rb.out());
+    HIP_TRY(launch_ring(ra, ctx->stream));
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if (res->pending) {
+      std::vector<uint32_t> st(n_q);
+      uint32_t any = 0u;
+      for (uint32_t q = 0; q < n_q; ++q) any |= st[q] = ra.out_status[q] & 0xffu;
+      if (any) {  // nothing was merged
+        bool rerun = false;
+        if ((rc = handle_scan_status(ctx, res, st.data(), n_q, &rerun))) return rc;
+        ra.gate = nullptr;
+        HIP_TRY(launch_ring(ra, ctx->stream));
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+      }
+      res->pending = false;
+    }
+    return ring_status_error(ra.out_status, n_q);
+  }
   mrl_rerank_store* store = nullptr;
   void* scratch = nullptr;
   uint8_t* merged = nullptr;

@@ -283,3 +283,51 @@ def test_ring_merge_into_scan_shortlists(device, n_pending):
         _lib.check(_lib.lib.mrl_results_merge_ring(device.handle, res._h, _lib.fptr(bad), n_pending, 768))
     assert e.value.code == 3
     res.close()
+
+
+@pytest.mark.parametrize("dims", [1, 255, 256, 257, 515, 768])
+@pytest.mark.parametrize("n_pending", [1, 64, 65, 256, 257])
+def test_ring_search_pieces(device, dims, n_pending):
+    """Edges of the fused ring kernel's pieces (64 rows x 256 dims) and of the
+    count it takes (256 rows; one more goes through the store)."""
+    from mrl_index_amd import _lib
+    rng = np.random.default_rng(1000 * dims + n_pending)
+    pending = rng.standard_normal((n_pending, dims)).astype(np.float32)
+    queries = rng.standard_normal((5, dims)).astype(np.float32)
+    loc = np.zeros((5, n_pending), dtype=np.uint64)
+    sc = np.zeros((5, n_pending), dtype=np.float32)
+    cnt = np.zeros(5, dtype=np.uint32)
+    _lib.check(_lib.lib.mrl_ring_search(device.handle, _lib.addr(pending), n_pending, dims, _lib.addr(queries), 5,
+                                        n_pending, _lib.addr(loc), _lib.addr(sc), _lib.addr(cnt)))
+    for q in range(5):
+        wl, ws = ora.ring_search_exact(pending, queries[q], n_pending)
+        assert np.array_equal(loc[q], wl) and np.array_equal(sc[q].view(np.uint32), ws.view(np.uint32))
+
+
+@pytest.mark.parametrize("alpha,w_s4,dense", [(1.0, 0.2, False), (0.8, 3.0, True)])
+def test_ring_merge_behind_an_unfetched_scan(device, alpha, w_s4, dense):
+    """The merge enqueued right behind a scan equals the merge of the fetched
+    scan, also when queries of the scan are re-run by the host (dense: bounds
+    that are not admissible) before anything may be merged."""
+    from mrl_index_amd import _lib
+    rng = np.random.default_rng(77)
+    rows = normalized(rng, 64 * 320 - 9, 768)
+    qs = (rows[rng.integers(0, rows.shape[0], 9)] + 0.01 * rng.standard_normal((9, 768))).astype(np.float32)
+    pending = np.ascontiguousarray(np.repeat(qs, 7, axis=0) + np.float32(0.3) * normalized(rng, 63, 768))
+    fit = m.EdenFit.fit_prefix(rows[:4096], 4, 1)
+    ix = m.DeviceIndex.upload(m.encode_corpus(rows, 8, fit), device)
+    plan = m.QueryPlan.from_query_eden(qs, 768, fit, device)
+    cfg = m.ScanConfig(shortlist_cand=48, cs_tolerance=alpha, stratum4_weight=w_s4)
+    out = []
+    for fetch_first in (True, False):
+        res = m.DeviceResults(9, 48, device)
+        res.scan(ix, plan, cfg)
+        if fetch_first:
+            assert (res.fetch().stats.reruns_dense > 0) == dense
+        _lib.check(_lib.lib.mrl_results_merge_ring(device.handle, res._h, _lib.addr(pending), 63, 768))
+        out.append(res.fetch())
+        res.close()
+    a, b = out
+    assert np.array_equal(a.counts, b.counts) and np.array_equal(a.ids, b.ids)
+    assert np.array_equal(a.scores.view(np.uint32), b.scores.view(np.uint32))
+    assert np.any((a.ids >> np.uint64(16)) == np.uint64(0xFFFFFFFF))
