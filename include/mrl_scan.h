@@ -499,7 +499,7 @@ int mrl_encode_corpus_device_clustered(mrl_ctx *ctx, const float *d_matrix, uint
 int mrl_device_alloc(mrl_ctx *ctx, size_t bytes, void **out);
 /* Pinned host memory for a caller's output arrays (no reference counterpart).
  * Where out_ids and out_scores of mrl_scan / mrl_results_fetch (out_rows and
- * out_scores of mrl_rerank_rows) lie in such blocks of the same context, the
+ * out_scores of mrl_rerank_rows / mrl_results_rerank) lie in such blocks of the same context, the
  * device writes them directly instead of through a staging copy; contents and
  * results are the same either way.  A block keeps its context alive until it
  * is freed; freed blocks are kept for the next mrl_host_alloc, at most 64 MiB

@@ -394,6 +394,8 @@ struct mrl_results {
   // rerank of the shortlists (allocated by the first mrl_results_rerank):
   // scores/rows scratch, sorted rows/scores, status
   void* d_rr = nullptr;
+  uint8_t* h_rr = nullptr;  // its mapped outputs (a pinned pool block)
+  size_t rr_bytes() const { return (size_t)std::max<uint32_t>(n_q, 1) * (8 + (size_t)k * 12); }
 };
 
 struct mrl_rerank_store {
@@ -1145,6 +1147,7 @@ static ScanParams make_params(const mrl_scan_config* cfg, const mrl_time_range* 
 static void results_free(mrl_results* r) {
   if (r->h_head) r->ctx->pin_pool.give(r->h_head, r->head_bytes());
   if (r->h_rows) r->ctx->pin_pool.give(r->h_rows, r->rows_bytes());
+  if (r->h_rr) r->ctx->pin_pool.give(r->h_rr, r->rr_bytes());
   dev_free(r->d_out);
   dev_free(r->d_cand_score);
   dev_free(r->d_cand_row);
@@ -2814,6 +2817,23 @@ static RerankBuffers rerank_carve(void* base, uint32_t n_q, uint32_t stride) {
   return b;
 }
 
+// b with its outputs in mapped host memory: the pinned block h, laid out as the
+// device block's head, or (rows and scores of n_q lists) the caller's arrays
+// where the device can write them.
+static RerankBuffers mapped_outputs(mrl_ctx* ctx, RerankBuffers b, uint8_t* h, uint32_t nq, uint32_t stride,
+                                    uint32_t n_q, uint64_t* out_rows, float* out_scores) {
+  const size_t n = (size_t)n_q * stride;
+  b.status = reinterpret_cast<uint32_t*>(h);
+  b.counts = b.status + nq;
+  b.out_rows = reinterpret_cast<uint64_t*>(h + (size_t)nq * 8);
+  b.out_scores = reinterpret_cast<float*>(h + (size_t)nq * 8 + (size_t)nq * stride * 8);
+  if (out_rows && out_scores && in_host_block(ctx, out_rows, n * 8) && in_host_block(ctx, out_scores, n * 4)) {
+    b.out_rows = out_rows;
+    b.out_scores = out_scores;
+  }
+  return b;
+}
+
 static int status_error(const uint32_t* st, uint32_t n) {
   uint32_t all = 0;
   for (uint32_t i = 0; i < n; ++i) all |= st[i] & 0xffu;
@@ -2866,9 +2886,9 @@ extern "C" int mrl_rerank_rows(mrl_ctx* ctx, const mrl_rerank_store* store, cons
     if (counts[q] > stride) return fail(MRL_ERR_INVALID_ARG, "count above stride");
   std::lock_guard<std::mutex> g(ctx->mu);
   HIP_TRY(hipSetDevice(ctx->device));
-  // One pool block on each side, laid out alike but for the device's scratch:
-  // the outputs (status, counts, rows, scores: one copy back), then the inputs
-  // [candidates][queries][counts] (one copy in).
+  // A device block [scratch][candidates][queries][counts] (the inputs arrive
+  // with one copy) and a pinned one [outputs][inputs]: the sort writes the
+  // outputs there, or into the caller's arrays where the device can.
   const size_t nc = (size_t)n_q * stride;
   const size_t qbytes = (size_t)n_q * dims * 4;
   const size_t in_at = (rerank_bytes(n_q, stride) + 15) & ~(size_t)15;
@@ -2882,32 +2902,20 @@ extern "C" int mrl_rerank_rows(mrl_ctx* ctx, const mrl_rerank_store* store, cons
     memcpy(h + out_bytes, cand_rows, nc * 8);
     memcpy(h + out_bytes + nc * 8, queries, qbytes);
     memcpy(h + out_bytes + nc * 8 + qbytes, counts, (size_t)n_q * 4);
-  }
-  if (!rc) {
-    const RerankBuffers b = rerank_carve(base, n_q, stride);
+    const RerankBuffers b = mapped_outputs(ctx, rerank_carve(base, n_q, stride), h, n_q, stride, n_q, out_rows, out_scores);
     uint64_t* d_cand = reinterpret_cast<uint64_t*>(base + in_at);
     float* d_q = reinterpret_cast<float*>(base + in_at + nc * 8);
     uint32_t* d_counts = reinterpret_cast<uint32_t*>(base + in_at + nc * 8 + qbytes);
     hipError_t e = hipMemcpyAsync(d_cand, h + out_bytes, in_bytes, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) rc = enqueue_rerank(ctx, store, d_q, n_q, d_cand, 0, d_counts, stride, b);
-    const bool direct = in_host_block(ctx, out_rows, nc * 8) && in_host_block(ctx, out_scores, nc * 4);
-    if (e == hipSuccess && !rc) {
-      if (direct) {
-        e = hipMemcpyAsync(out_rows, b.out_rows, nc * 8, hipMemcpyDeviceToHost, ctx->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(out_scores, b.out_scores, nc * 4, hipMemcpyDeviceToHost, ctx->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(h, b.status, (size_t)n_q * 8, hipMemcpyDeviceToHost, ctx->stream);
-      } else {
-        e = hipMemcpyAsync(h, b.status, rerank_out_bytes(n_q, stride), hipMemcpyDeviceToHost, ctx->stream);
-      }
-    }
     const hipError_t es = hipStreamSynchronize(ctx->stream);
     if (e == hipSuccess) e = es;
     if (!rc && e != hipSuccess) rc = fail(MRL_ERR_HIP, std::string("rerank: ") + hipGetErrorString(e));
-    if (!rc && !direct) {
-      memcpy(out_rows, h + (size_t)n_q * 8, nc * 8);
-      memcpy(out_scores, h + (size_t)n_q * 8 + nc * 8, nc * 4);
+    if (!rc) rc = status_error(b.status, n_q);
+    if (!rc && b.out_rows != out_rows) {
+      memcpy(out_rows, b.out_rows, nc * 8);
+      memcpy(out_scores, b.out_scores, nc * 4);
     }
-    if (!rc) rc = status_error(reinterpret_cast<const uint32_t*>(h), n_q);
   }
   if (base) ctx->dev_pool.give(base, in_at + in_bytes);
   if (h) ctx->pin_pool.give(h, out_bytes + in_bytes);
@@ -2932,34 +2940,32 @@ extern "C" int mrl_results_rerank(mrl_ctx* ctx, mrl_results* res, const mrl_rera
     res->d_rr = nullptr;
     return fail(MRL_ERR_OUT_OF_MEMORY, "rerank buffers");
   }
-  const RerankBuffers b = rerank_carve(res->d_rr, nq, K);
-  const size_t n = (size_t)nq * K;
-  uint8_t* h = host_stage(ctx, rerank_out_bytes(nq, K));
-  if (!h) return fail(MRL_ERR_OUT_OF_MEMORY, "pinned staging buffer");
-  // The rerank is enqueued right behind the scan; the scan's status rides
-  // along in bits 8.. of the rerank status, so one read-back serves both.
+  if (!res->h_rr) res->h_rr = ctx->pin_pool.take(res->rr_bytes());
+  if (!res->h_rr) return fail(MRL_ERR_OUT_OF_MEMORY, "pinned rerank buffer");
+  const RerankBuffers b =
+      mapped_outputs(ctx, rerank_carve(res->d_rr, nq, K), res->h_rr, nq, K, n_q, out_rows, out_scores);
+  // The rerank is enqueued right behind the scan, its sort writes to host
+  // memory, and the scan's status rides along in bits 8.. of the rerank
+  // status, so one wait serves both.
   auto run = [&](const uint32_t* scan_status) -> int {
     int rc = enqueue_rerank(ctx, store, plans->d_queries, n_q, res->d_ids, 1, res->d_counts, K, b, scan_status);
-    if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(h, b.status, (size_t)nq * 8 + (size_t)n_q * K * 8, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipMemcpyAsync(h + (size_t)nq * 8 + n * 8, b.out_scores, (size_t)n_q * K * 4, hipMemcpyDeviceToHost,
-                           ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-    return MRL_OK;
+    const hipError_t e = hipStreamSynchronize(ctx->stream);  // also on an error: the arrays may be the caller's
+    if (!rc && e != hipSuccess) rc = fail(MRL_ERR_HIP, std::string("rerank: ") + hipGetErrorString(e));
+    return rc;
   };
   const bool pend = res->pending && res->last_index && res->last_index->n_blocks;
   int rc = run(pend ? res->d_status : nullptr);
   if (rc) return rc;
-  const uint32_t* st = reinterpret_cast<const uint32_t*>(h);
+  const uint32_t* st = b.status;
   std::vector<uint32_t> scan_st(n_q);
   for (uint32_t q = 0; q < n_q; ++q) scan_st[q] = st[q] >> 8;
   bool rerun = false;
   if ((rc = handle_scan_status(ctx, res, scan_st.data(), n_q, &rerun))) return rc;
   if (rerun && (rc = run(nullptr))) return rc;
   if ((rc = status_error(st, n_q))) return rc;
-  if (out_rows) memcpy(out_rows, h + (size_t)nq * 8, (size_t)n_q * K * 8);
-  if (out_scores) memcpy(out_scores, h + (size_t)nq * 8 + n * 8, (size_t)n_q * K * 4);
-  if (out_counts) memcpy(out_counts, h + (size_t)nq * 4, (size_t)n_q * 4);
+  if (out_rows && out_rows != b.out_rows) memcpy(out_rows, b.out_rows, (size_t)n_q * K * 8);
+  if (out_scores && out_scores != b.out_scores) memcpy(out_scores, b.out_scores, (size_t)n_q * K * 4);
+  if (out_counts) memcpy(out_counts, b.counts, (size_t)n_q * 4);
   return MRL_OK;
 }
 

@@ -407,7 +407,8 @@ struct RerankArgs {
   int32_t cand_ids;
   float* score;             // scratch [n_q][stride]
   uint64_t* row;            // scratch [n_q][stride]
-  uint64_t* out_rows;       // [n_q][stride], sorted
+  uint64_t* out_rows;       // [n_q][stride], sorted, zeros past the list (this and the outputs below may be mapped
+                            // host memory)
   float* out_scores;
   uint32_t* status;         // [n_q]: bit 0 NaN score, bit 1 row out of range
   uint32_t* out_counts;     // [n_q] or null: entries written per query (ring hits excluded)
@@ -429,30 +430,6 @@ struct RingMergeArgs {
   uint64_t* out_ids;          // [n_q][k]
   float* out_scores;
   uint32_t* out_counts;       // [n_q]
-};
-
-// Ring search, and its merge into the scan shortlists, of up to kRingFused
-// pending rows in one launch (the ring flushes at 64): one workgroup scores
-// the rows for one query, sorts them and merges or writes them.
-constexpr uint32_t kRingFused = 256;
-struct RingArgs {
-  const float* rows;          // [n_ring][dims] pending rows, row-major
-  const float* queries;       // [n_q][dims]
-  uint32_t n_ring;            // 1 .. kRingFused
-  uint32_t dims;
-  uint32_t n_q;
-  // merge (ids != null): the shortlists, merged in place, and their status;
-  // with gate set nothing is merged when any query's status is not 0
-  uint32_t k;
-  uint64_t* ids;              // [n_q][k]
-  float* scores;
-  uint32_t* counts;           // [n_q]
-  const uint32_t* gate;       // [n_q] or null
-  uint32_t* out_status;       // [n_q] (may be mapped host memory): gate's value, bit 8: a NaN ring score
-  // search (ids == null): the first `keep` hits of each query
-  uint32_t keep;
-  uint64_t* out_local;        // [n_q][keep]
-  float* out_scores;
 };
 
 // Ring search, and its merge into the scan shortlists, of up to kRingFused
@@ -596,7 +573,6 @@ hipError_t launch_rerank_store(const float* rows, uint64_t n_rows, int precision
                                hipStream_t s);
 hipError_t launch_rerank(const RerankArgs& a, hipStream_t s, const LaunchEvents& ev_score = {},
                          const LaunchEvents& ev_sort = {});
-hipError_t launch_ring(const RingArgs& a, hipStream_t s, const LaunchEvents& ev = {});
 hipError_t launch_ring(const RingArgs& a, hipStream_t s, const LaunchEvents& ev = {});
 hipError_t launch_ring_merge(const RingMergeArgs& a, hipStream_t s, const LaunchEvents& ev = {});
 
