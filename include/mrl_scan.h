@@ -178,7 +178,8 @@ size_t mrl_query_plan_size(void);
  * freed with the last of them.  After mrl_ctx_destroy the handle may not be
  * passed to any call (its objects' own destroy calls remain valid).  Memory
  * from mrl_device_alloc is freed with mrl_device_free(ctx, ...) before
- * mrl_ctx_destroy.  Destroy calls wait for the context's stream first. */
+ * mrl_ctx_destroy.  Destroy calls wait for the work that still uses the
+ * object. */
 int mrl_ctx_create(int device, mrl_ctx **out);
 void mrl_ctx_destroy(mrl_ctx *ctx);
 int mrl_ctx_synchronize(mrl_ctx *ctx);

@@ -73,6 +73,7 @@ static const size_t kPoolKeep = (size_t)64 << 20;
 struct BlockPool {
   explicit BlockPool(bool pinned_) : pinned(pinned_) {}
   const bool pinned;
+  hipStream_t stream = nullptr;  // the only stream whose work uses the device blocks
   std::mutex mu;
   std::vector<std::pair<uint8_t*, size_t>> free_blocks;
   size_t kept = 0;
@@ -81,7 +82,14 @@ struct BlockPool {
     while (r < bytes) r <<= 1;
     return r;
   }
-  void release(uint8_t* p) const { (void)(pinned ? hipHostFree(p) : hipFree(p)); }
+  void release(uint8_t* p) const {
+    if (pinned) {
+      (void)hipHostFree(p);
+      return;
+    }
+    (void)hipStreamSynchronize(stream);
+    (void)hipFree(p);
+  }
   // null: out of memory
   uint8_t* take(size_t bytes) {
     bytes = rounded(bytes);
@@ -98,14 +106,16 @@ struct BlockPool {
     }
     for (int attempt = 0; attempt < 2; ++attempt) {
       void* p = nullptr;
-      if ((pinned ? hipHostMalloc(&p, bytes, hipHostMallocDefault) : hipMalloc(&p, bytes)) == hipSuccess)
+      if ((pinned ? hipHostMalloc(&p, bytes, hipHostMallocCoherent) : hipMalloc(&p, bytes)) == hipSuccess)
         return static_cast<uint8_t*>(p);
       (void)hipGetLastError();  // do not leave the failure for the next launch check
       trim();
     }
     return nullptr;
   }
-  // The device no longer uses p (taken with this size).
+  // Gives back p (taken with this size): a pinned block the device no longer
+  // uses; a device block that only work already on the stream uses, since the
+  // next taker's work comes after it on the same stream.
   void give(void* p, size_t bytes) {
     if (!p) return;
     bytes = rounded(bytes);
@@ -332,6 +342,7 @@ struct mrl_plans {
   size_t d_bytes = 0;
   uint8_t* h_in = nullptr;     // pinned pool block the host inputs are copied from
   size_t h_bytes = 0;
+  mutable bool copied = false; // a scan that used the inputs is known to be done
   // The plans are built lazily: by the next call that reads them (flush_plans),
   // or inside a one-query sampling pass (k_scan's fused plan).
   mutable bool pending = false;
@@ -426,6 +437,7 @@ extern "C" int mrl_ctx_create(int device, mrl_ctx** out) {
   std::unique_ptr<mrl_ctx> c(new mrl_ctx());
   c->device = device;
   HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+  c->dev_pool.stream = c->stream;
   // IEEE constants the reference computes with the same f32 operations.
   c->consts.inv_sqrt64 = 1.0f / sqrtf(64.0f);
   c->consts.inv_sqrt128 = 1.0f / sqrtf(128.0f);
@@ -522,6 +534,33 @@ static bool in_host_block(mrl_ctx* ctx, const void* p, size_t bytes) {
   if (it == ctx->host_blocks.begin()) return false;
   --it;
   return (uintptr_t)p + bytes <= it->first + it->second;
+}
+
+// Waits for an enqueued launch that stores n status words.  Up to
+// kSignalMaxQueries of them are signalled (signal_status; the caller set them
+// to kStatusPending before the launch): polls them for up to 2 ms, then waits
+// for the stream, which also reports a launch that failed.
+static int wait_status(mrl_ctx* ctx, const uint32_t* status, uint32_t n) {
+  if (n > kSignalMaxQueries) {
+    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    return e == hipSuccess ? MRL_OK : fail(MRL_ERR_HIP, std::string("wait: ") + hipGetErrorString(e));
+  }
+  const auto t0 = std::chrono::steady_clock::now();
+  for (uint32_t q = 0; q < n; ++q) {
+    uint32_t spins = 0;
+    while (__atomic_load_n(status + q, __ATOMIC_ACQUIRE) == kStatusPending) {
+      __builtin_ia32_pause();
+      if ((++spins & 255u) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+        const hipError_t e = hipStreamSynchronize(ctx->stream);
+        if (e != hipSuccess) return fail(MRL_ERR_HIP, std::string("wait: ") + hipGetErrorString(e));
+        for (uint32_t i = q; i < n; ++i)
+          if (__atomic_load_n(status + i, __ATOMIC_ACQUIRE) == kStatusPending)
+            return fail(MRL_ERR_HIP, "a launch ended without its status");
+        return MRL_OK;
+      }
+    }
+  }
+  return MRL_OK;
 }
 
 extern "C" int mrl_ctx_synchronize(mrl_ctx* ctx) {
@@ -1049,10 +1088,12 @@ static int plans_build_impl(mrl_ctx* ctx, const float* queries, bool on_device, 
     if (n_q) memcpy(hf + 192, queries, qbytes);
     e = hipMemcpyAsync(d_in, hf, in_bytes, hipMemcpyHostToDevice, ctx->stream);
   } else {
+    // (the pool block may still be in use by work on the stream; the copy below runs on another)
+    e = hipStreamSynchronize(ctx->stream);
     float means[192] = {0};
     if (eden) memcpy(means, eden->mean, 64 * sizeof(float));
     if (eden_mid) memcpy(means + 64, eden_mid->mean, 128 * sizeof(float));
-    e = hipMemcpy(d_in, means, sizeof(means), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(d_in, means, sizeof(means), hipMemcpyHostToDevice);
     if (e == hipSuccess && n_q) e = hipMemcpyAsync(d_in + 192, queries, qbytes, hipMemcpyDeviceToDevice, ctx->stream);
   }
   if (e != hipSuccess) {
@@ -1111,7 +1152,7 @@ extern "C" void mrl_plans_destroy(mrl_plans* plans) {
   if (!plans) return;
   mrl_ctx* ctx = plans->ctx;
   (void)hipSetDevice(ctx->device);
-  (void)hipStreamSynchronize(ctx->stream);
+  if (!plans->copied) (void)hipStreamSynchronize(ctx->stream);  // the input copy may still read h_in
   ctx->dev_pool.give(plans->d_block, plans->d_bytes);
   ctx->pin_pool.give(plans->h_in, plans->h_bytes);
   delete plans;
@@ -1275,10 +1316,11 @@ struct PassBuffers {
 
 // A selection with mapped outputs sums the counters for the host, which takes
 // the re-run counts from the statuses; one on the device counts them itself.
-static void set_select_stats(SelectArgs* sa, const PassBuffers& pb, unsigned long long* stats) {
+static void set_select_stats(SelectArgs* sa, const PassBuffers& pb, unsigned long long* stats, uint32_t n_q) {
   if (pb.stats_sum && stats) {
     sa->stats_src = stats;
     sa->stats_sum = pb.stats_sum;
+    sa->signal = n_q <= kSignalMaxQueries ? 1u : 0u;
   } else {
     sa->stats = stats;
   }
@@ -1667,7 +1709,7 @@ static int enqueue_scan_mma(mrl_ctx* ctx, mrl_index* ix, const mrl_plans* plans,
   sa.out_ids = pb.out_ids;
   sa.out_scores = pb.out_scores;
   sa.out_counts = pb.out_counts;
-  set_select_stats(&sa, pb, stats);
+  set_select_stats(&sa, pb, stats, n_q);
   sa.hist = sampled ? pb.hist : nullptr;
   sa.tau_final = pb.tau_hi;
   sa.tau_safe = pb.tau;
@@ -1785,7 +1827,7 @@ static int enqueue_scan(mrl_ctx* ctx, mrl_index* ix, const mrl_plans* plans, uin
   sa.out_ids = pb.out_ids;
   sa.out_scores = pb.out_scores;
   sa.out_counts = pb.out_counts;
-  set_select_stats(&sa, pb, stats);
+  set_select_stats(&sa, pb, stats, n_q);
   sa.hist = sampled ? pb.hist : nullptr;
   sa.tau_final = pb.tau_hi;
   sa.tau_safe = pb.tau;
@@ -2156,8 +2198,10 @@ static int scan_mapped(mrl_ctx* ctx, const mrl_index* index, const mrl_plans* pl
   res->o_ids = direct ? out_ids : reinterpret_cast<uint64_t*>(res->h_rows);
   res->o_scores = direct ? out_scores : reinterpret_cast<float*>(res->h_rows + nq * K * 8);
   bool sampled, rerun;
+  for (uint32_t q = 0; q < n_q; ++q) res->o_status[q] = kStatusPending;
   rc = enqueue_scan_into(ctx, index, plans, cfg, time, res, K, &sampled);
-  if (!rc && hipStreamSynchronize(ctx->stream) != hipSuccess) rc = fail(MRL_ERR_HIP, "scan");
+  if (!rc && index->n_blocks) rc = wait_status(ctx, res->o_status, n_q);
+  if (!rc && n_q && index->n_blocks) plans->copied = true;
   unsigned long long st[kStatCount];
   memcpy(st, res->stats_seen, sizeof(st));
   if (!rc && n_q && index->n_blocks) {
@@ -2845,8 +2889,12 @@ static int status_error(const uint32_t* st, uint32_t n) {
 // Enqueue score + sort.  Caller holds the lock.
 static int enqueue_rerank(mrl_ctx* ctx, const mrl_rerank_store* st, const float* d_queries, uint32_t n_q,
                           const uint64_t* d_cand, int cand_ids, const uint32_t* d_counts, uint32_t stride,
-                          const RerankBuffers& b, const uint32_t* d_scan_status = nullptr) {
+                          const RerankBuffers& b, const uint32_t* d_scan_status = nullptr, bool signal = false) {
   RerankArgs a{};
+  signal = signal && n_q <= kSignalMaxQueries;
+  a.signal = signal ? 1u : 0u;
+  if (signal)
+    for (uint32_t q = 0; q < n_q; ++q) b.status[q] = kStatusPending;
   a.data = st->d_data;
   a.scales = st->d_scales;
   a.n_rows = st->n_rows;
@@ -2907,10 +2955,10 @@ extern "C" int mrl_rerank_rows(mrl_ctx* ctx, const mrl_rerank_store* store, cons
     float* d_q = reinterpret_cast<float*>(base + in_at + nc * 8);
     uint32_t* d_counts = reinterpret_cast<uint32_t*>(base + in_at + nc * 8 + qbytes);
     hipError_t e = hipMemcpyAsync(d_cand, h + out_bytes, in_bytes, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) rc = enqueue_rerank(ctx, store, d_q, n_q, d_cand, 0, d_counts, stride, b);
-    const hipError_t es = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) e = es;
-    if (!rc && e != hipSuccess) rc = fail(MRL_ERR_HIP, std::string("rerank: ") + hipGetErrorString(e));
+    if (e == hipSuccess) rc = enqueue_rerank(ctx, store, d_q, n_q, d_cand, 0, d_counts, stride, b, nullptr, true);
+    else rc = fail(MRL_ERR_HIP, std::string("rerank: ") + hipGetErrorString(e));
+    if (!rc) rc = wait_status(ctx, b.status, n_q);
+    if (rc) (void)hipStreamSynchronize(ctx->stream);  // nothing may still use the blocks
     if (!rc) rc = status_error(b.status, n_q);
     if (!rc && b.out_rows != out_rows) {
       memcpy(out_rows, b.out_rows, nc * 8);
@@ -2948,9 +2996,10 @@ extern "C" int mrl_results_rerank(mrl_ctx* ctx, mrl_results* res, const mrl_rera
   // memory, and the scan's status rides along in bits 8.. of the rerank
   // status, so one wait serves both.
   auto run = [&](const uint32_t* scan_status) -> int {
-    int rc = enqueue_rerank(ctx, store, plans->d_queries, n_q, res->d_ids, 1, res->d_counts, K, b, scan_status);
-    const hipError_t e = hipStreamSynchronize(ctx->stream);  // also on an error: the arrays may be the caller's
-    if (!rc && e != hipSuccess) rc = fail(MRL_ERR_HIP, std::string("rerank: ") + hipGetErrorString(e));
+    int rc = enqueue_rerank(ctx, store, plans->d_queries, n_q, res->d_ids, 1, res->d_counts, K, b, scan_status, true);
+    if (!rc) rc = wait_status(ctx, b.status, n_q);
+    if (rc) (void)hipStreamSynchronize(ctx->stream);  // the arrays may be the caller's
+    else plans->copied = true;
     return rc;
   };
   const bool pend = res->pending && res->last_index && res->last_index->n_blocks;
@@ -2993,8 +3042,7 @@ static int check_ring_args(const float* pending, uint32_t n_pending, uint32_t di
 }
 
 // The fused ring kernel's call: the pending rows (and, for a search, the
-// queries) go to a pool block with one copy; `run` enqueues the launches and
-// waits.  Caller holds the lock.  h: pinned, [inputs][out_bytes of outputs].
+// queries) go to a pool block with one copy; `run` launches and waits.  Caller holds the lock.  h: pinned, [inputs][out_bytes of outputs].
 struct RingBlocks {
   mrl_ctx* ctx;
   size_t in_bytes, out_bytes;
@@ -3004,6 +3052,11 @@ struct RingBlocks {
     h = d ? ctx->pin_pool.take(in_bytes + out_bytes) : nullptr;
   }
   uint8_t* out() const { return h + in_bytes; }
+  int run(const RingArgs& a) {
+    HIP_TRY(launch_ring(a, ctx->stream));
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    return MRL_OK;
+  }
   ~RingBlocks() {
     (void)hipStreamSynchronize(ctx->stream);
     if (d) ctx->dev_pool.give(d, in_bytes);
@@ -3050,8 +3103,7 @@ extern "C" int mrl_ring_search(mrl_ctx* ctx, const float* pending, uint32_t n_pe
     ra.out_local = reinterpret_cast<uint64_t*>(rb.out());
     ra.out_scores = reinterpret_cast<float*>(rb.out() + nk * 8);
     ra.out_status = reinterpret_cast<uint32_t*>(rb.out() + nk * 12);
-    HIP_TRY(launch_ring(ra, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if ((rc = rb.run(ra))) return rc;
     memcpy(out_local, ra.out_local, nk * 8);
     memcpy(out_scores, ra.out_scores, nk * 4);
     for (uint32_t q = 0; q < n_q; ++q) out_counts[q] = keep;
@@ -3123,8 +3175,7 @@ extern "C" int mrl_results_merge_ring(mrl_ctx* ctx, mrl_results* res, const floa
     ra.counts = res->d_counts;
     ra.gate = res->pending ? res->d_status : nullptr;
     ra.out_status = reinterpret_cast<uint32_t*>(rb.out());
-    HIP_TRY(launch_ring(ra, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if ((rc = rb.run(ra))) return rc;
     if (res->pending) {
       std::vector<uint32_t> st(n_q);
       uint32_t any = 0u;
@@ -3133,8 +3184,7 @@ extern "C" int mrl_results_merge_ring(mrl_ctx* ctx, mrl_results* res, const floa
         bool rerun = false;
         if ((rc = handle_scan_status(ctx, res, st.data(), n_q, &rerun))) return rc;
         ra.gate = nullptr;
-        HIP_TRY(launch_ring(ra, ctx->stream));
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        if ((rc = rb.run(ra))) return rc;
       }
       res->pending = false;
     }

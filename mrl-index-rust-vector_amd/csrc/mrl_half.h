@@ -1,4 +1,4 @@
-// mrl_half.h -- IEEE binary16 conversions shared by the device code.
+// mrl_half.h -- IEEE binary16 conversions and the host signal, shared by the device code.
 #pragma once
 
 #include <stdint.h>
@@ -39,6 +39,16 @@ __device__ __forceinline__ uint32_t f32_to_f16(float f) {
   uint32_t out = base + kept;
   if (rem > halfway || (rem == halfway && (kept & 1u))) out += 1u;
   return out & 0xffffu;
+}
+
+// Stores a query's status in host memory once everything its workgroup wrote
+// is visible there (called by one thread after the workgroup's barrier).  The
+// host polls the word: the wait ends about 5 us before the stream's own
+// completion signal would wake a hipStreamSynchronize (an empty kernel: 8.0
+// against 13.6 us).
+__device__ __forceinline__ void signal_status(uint32_t* status, uint32_t value) {
+  __threadfence_system();
+  __hip_atomic_store(status, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace mrl

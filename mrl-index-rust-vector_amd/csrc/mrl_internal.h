@@ -357,6 +357,10 @@ struct SelectArgs {
   // re-run counts (which status holds); null: not asked for.
   const unsigned long long* stats_src;
   unsigned long long* stats_sum;
+  // The host waits for the statuses (mapped host memory, preset to
+  // kStatusPending): a query's is stored last, after its other outputs are
+  // visible to the host.
+  uint32_t signal;
   // Gated re-run: query q is selected only if bit 2 of gate[q] is set
   // (gate is the status array this launch rewrites); null: every query.
   const uint32_t* gate;
@@ -413,6 +417,7 @@ struct RerankArgs {
   uint32_t* status;         // [n_q]: bit 0 NaN score, bit 1 row out of range
   uint32_t* out_counts;     // [n_q] or null: entries written per query (ring hits excluded)
   const uint32_t* scan_status;  // [n_q] or null: copied into status bits 8..10
+  uint32_t signal;          // as SelectArgs::signal
 };
 
 // Ring merge (mrl_rerank.hip): push the sorted ring hits of each query into
@@ -512,6 +517,17 @@ struct BoundScanArgs {
   uint32_t stride;
   float* out_bound;           // diagnostic [n_q][n_blocks] bounds (NaN: unbounded block), or null
 };
+
+// What the host sets a status word to before it waits for the launch that
+// stores it (signal_status).
+constexpr uint32_t kStatusPending = 0xffffffffu;
+// Batches up to this size end with signalled statuses: each signal's
+// system-scope release writes back its XCD's L2, which costs what the earlier
+// wake-up saves once many workgroups do it (us per call, signalled against a
+// stream wait: 1 query 62.5 / 66.3, scan + rerank of 32 queries 144.3 / 163.2,
+// 64 queries 270.5 / 270.2, 256 queries 293.5 / 294.8, rerank of 256 lists
+// 154.8 / 143.3).
+constexpr uint32_t kSignalMaxQueries = 32;
 
 // Launchers (mrl_kernels.hip).
 // Optional start/stop events written by the dispatch itself (kernel-only

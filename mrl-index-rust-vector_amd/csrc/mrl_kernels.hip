@@ -2355,6 +2355,7 @@ __global__ __launch_bounds__(kSelThreads) void k_select(SelectArgs a) {
   if (tid < (int)a.nseg) a.seg_count[(uint64_t)q * a.nseg + tid] = 0u;
   if (a.hist)
     for (int i = tid; i < kHistBins; i += kSelThreads) a.hist[(uint64_t)q * kHistBins + i] = 0u;
+  if (a.signal) __syncthreads();  // every thread's outputs before the status
   if (tid == 0) {
     // Fewer than K candidates above a floor tighter than the safe one: the
     // top K may lie below it, so the final pass is re-run at the safe floor.
@@ -2367,8 +2368,10 @@ __global__ __launch_bounds__(kSelThreads) void k_select(SelectArgs a) {
     const uint32_t short_f = (!short_k && keep < K && s_fl[2] > -INFINITY) ? 8u : 0u;
     a.out_counts[q] = keep;
     if (a.floor_record) a.floor_record[q] = s_fl[2];
-    a.status[q] = (a.err[q] & 1u) | s_misc[7] | short_k | short_f;
+    const uint32_t status = (a.err[q] & 1u) | s_misc[7] | short_k | short_f;
     a.err[q] = 0u;
+    if (a.signal) signal_status(a.status + q, status);
+    else a.status[q] = status;
     if (a.stats && (short_k | short_f | s_misc[7])) {
       unsigned long long* st = a.stats + (q % (uint32_t)kStatCopies) * kStatCount;
       if (short_k) atomicAdd(st + kStatRerunSafe, 1ull);
