@@ -536,6 +536,16 @@ static bool in_host_block(mrl_ctx* ctx, const void* p, size_t bytes) {
   return (uintptr_t)p + bytes <= it->first + it->second;
 }
 
+// Copies between device memory and pinned host memory on the stream.
+static hipError_t copy_on(hipStream_t s, void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+  if (bytes > kCopyKernelMax || bytes % 4) return hipMemcpyAsync(dst, src, bytes, kind, s);
+  CopyArgs c{};
+  c.src[0] = src;
+  c.dst[0] = dst;
+  c.bytes[0] = bytes;
+  return launch_copy(c, s);
+}
+
 // Waits for an enqueued launch that stores n status words.  Up to
 // kSignalMaxQueries of them are signalled (signal_status; the caller set them
 // to kStatusPending before the launch): polls them for up to 2 ms, then waits
@@ -1086,7 +1096,7 @@ static int plans_build_impl(mrl_ctx* ctx, const float* queries, bool on_device, 
     if (eden) memcpy(hf, eden->mean, 64 * sizeof(float));
     if (eden_mid) memcpy(hf + 64, eden_mid->mean, 128 * sizeof(float));
     if (n_q) memcpy(hf + 192, queries, qbytes);
-    e = hipMemcpyAsync(d_in, hf, in_bytes, hipMemcpyHostToDevice, ctx->stream);
+    e = copy_on(ctx->stream, d_in, hf, in_bytes, hipMemcpyHostToDevice);
   } else {
     // (the pool block may still be in use by work on the stream; the copy below runs on another)
     e = hipStreamSynchronize(ctx->stream);
@@ -2065,9 +2075,15 @@ static int read_back(mrl_ctx* ctx, mrl_results* res, uint32_t n_q, uint8_t** out
   if (ids) {
     uint8_t* h = host_stage(ctx, head);
     if (!h) return fail(MRL_ERR_OUT_OF_MEMORY, "pinned staging buffer");
-    hipError_t e = hipMemcpyAsync(ids, res->d_ids, n_q * K * 8, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(scores, res->d_scores, n_q * K * 4, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(h, res->d_out, head, hipMemcpyDeviceToHost, ctx->stream);
+    hipError_t e;
+    if (n_q * K * 8 <= kCopyKernelMax) {
+      const CopyArgs c{{res->d_ids, res->d_scores, res->d_out}, {ids, scores, h}, {n_q * K * 8, n_q * K * 4, head}};
+      e = launch_copy(c, ctx->stream);
+    } else {
+      e = hipMemcpyAsync(ids, res->d_ids, n_q * K * 8, hipMemcpyDeviceToHost, ctx->stream);
+      if (e == hipSuccess) e = hipMemcpyAsync(scores, res->d_scores, n_q * K * 4, hipMemcpyDeviceToHost, ctx->stream);
+      if (e == hipSuccess) e = hipMemcpyAsync(h, res->d_out, head, hipMemcpyDeviceToHost, ctx->stream);
+    }
     const hipError_t es = hipStreamSynchronize(ctx->stream);  // also on an error: the arrays are the caller's
     if (e != hipSuccess || es != hipSuccess)
       return fail(MRL_ERR_HIP, std::string("results copy: ") + hipGetErrorString(e != hipSuccess ? e : es));
@@ -2076,7 +2092,11 @@ static int read_back(mrl_ctx* ctx, mrl_results* res, uint32_t n_q, uint8_t** out
   }
   uint8_t* h = host_stage(ctx, res->out_bytes);
   if (!h) return fail(MRL_ERR_OUT_OF_MEMORY, "pinned staging buffer");
-  if (n_q == nq) {
+  if (res->out_bytes <= kCopyKernelMax) {
+    const size_t at = head + nq * K * 8;
+    const CopyArgs c{{res->d_out, res->d_out + at, nullptr}, {h, h + at, nullptr}, {head + n_q * K * 8, n_q * K * 4, 0}};
+    HIP_TRY(launch_copy(c, ctx->stream));
+  } else if (n_q == nq) {
     HIP_TRY(hipMemcpyAsync(h, res->d_out, res->out_bytes, hipMemcpyDeviceToHost, ctx->stream));
   } else {
     HIP_TRY(hipMemcpyAsync(h, res->d_out, head + n_q * K * 8, hipMemcpyDeviceToHost, ctx->stream));
@@ -2954,7 +2974,7 @@ extern "C" int mrl_rerank_rows(mrl_ctx* ctx, const mrl_rerank_store* store, cons
     uint64_t* d_cand = reinterpret_cast<uint64_t*>(base + in_at);
     float* d_q = reinterpret_cast<float*>(base + in_at + nc * 8);
     uint32_t* d_counts = reinterpret_cast<uint32_t*>(base + in_at + nc * 8 + qbytes);
-    hipError_t e = hipMemcpyAsync(d_cand, h + out_bytes, in_bytes, hipMemcpyHostToDevice, ctx->stream);
+    hipError_t e = copy_on(ctx->stream, d_cand, h + out_bytes, in_bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) rc = enqueue_rerank(ctx, store, d_q, n_q, d_cand, 0, d_counts, stride, b, nullptr, true);
     else rc = fail(MRL_ERR_HIP, std::string("rerank: ") + hipGetErrorString(e));
     if (!rc) rc = wait_status(ctx, b.status, n_q);
@@ -3092,7 +3112,7 @@ extern "C" int mrl_ring_search(mrl_ctx* ctx, const float* pending, uint32_t n_pe
     if (!rb.h) return fail(MRL_ERR_OUT_OF_MEMORY, "ring search buffers");
     memcpy(rb.h, pending, pbytes);
     memcpy(rb.h + pbytes, queries, (size_t)n_q * dims * 4);
-    HIP_TRY(hipMemcpyAsync(rb.d, rb.h, pbytes + (size_t)n_q * dims * 4, hipMemcpyHostToDevice, ctx->stream));
+    HIP_TRY(copy_on(ctx->stream, rb.d, rb.h, pbytes + (size_t)n_q * dims * 4, hipMemcpyHostToDevice));
     RingArgs ra{};
     ra.rows = reinterpret_cast<const float*>(rb.d);
     ra.queries = reinterpret_cast<const float*>(rb.d + pbytes);
@@ -3162,7 +3182,7 @@ extern "C" int mrl_results_merge_ring(mrl_ctx* ctx, mrl_results* res, const floa
     RingBlocks rb(ctx, pbytes, (size_t)n_q * 4);
     if (!rb.h) return fail(MRL_ERR_OUT_OF_MEMORY, "ring merge");
     memcpy(rb.h, pending, pbytes);
-    HIP_TRY(hipMemcpyAsync(rb.d, rb.h, pbytes, hipMemcpyHostToDevice, ctx->stream));
+    HIP_TRY(copy_on(ctx->stream, rb.d, rb.h, pbytes, hipMemcpyHostToDevice));
     RingArgs ra{};
     ra.rows = reinterpret_cast<const float*>(rb.d);
     ra.queries = plans->d_queries;

@@ -551,6 +551,19 @@ int scan_query_tile(uint32_t n_q);  // queries per workgroup of the non-tile ker
 uint32_t scan_grid(const ScanArgs& a, bool diag);
 hipError_t launch_scan(const ScanArgs& a, bool diag, hipStream_t s, const LaunchEvents& ev = {});
 hipError_t launch_select(const SelectArgs& a, uint32_t n_q, hipStream_t s, const LaunchEvents& ev = {});
+// Copies between device memory and mapped host memory on the call path, up to
+// three at once (bytes multiples of 4; 0: none).  Below kCopyKernelMax a
+// launch beats hipMemcpyAsync, which above 16 KB hands the copy to another
+// engine and orders it against the stream's kernels with signals (then + a
+// kernel + a wait, us: 100 KB in 15.0 / 19.6, out 14.5 / 21.7; 800 KB in
+// 31.4 / 32.0, out 26.8 / 34.0); larger copies leave the CUs free.
+constexpr size_t kCopyKernelMax = (size_t)1 << 20;
+struct CopyArgs {
+  const void* src[3];
+  void* dst[3];
+  uint64_t bytes[3];
+};
+hipError_t launch_copy(const CopyArgs& a, hipStream_t s);
 // Sets n words at p to v (a kernel, so that a caller may capture it in a graph).
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
 // Reads n uint4 at p (evicts the caches; the loads are kept alive by a store

@@ -4362,6 +4362,38 @@ hipError_t launch_scan(const ScanArgs& a, bool diag, hipStream_t s, const Launch
   return hipGetLastError();
 }
 
+// Copy blockIdx.y of a; 16 bytes a time where both ends allow it.
+__global__ __launch_bounds__(256) void k_copy(CopyArgs a) {
+  const uint64_t n = a.bytes[blockIdx.y];
+  const char* src = static_cast<const char*>(a.src[blockIdx.y]);
+  char* dst = static_cast<char*>(a.dst[blockIdx.y]);
+  const uint64_t t = (uint64_t)blockIdx.x * 256u + threadIdx.x, step = (uint64_t)gridDim.x * 256u;
+  const bool wide = ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15u) == 0;
+  const uint64_t n16 = wide ? n / 16u : 0u;
+  for (uint64_t i = t; i < n16; i += step) reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+  for (uint64_t i = 4u * n16 + t; i < n / 4u; i += step)
+    reinterpret_cast<uint32_t*>(dst)[i] = reinterpret_cast<const uint32_t*>(src)[i];
+}
+
+hipError_t launch_copy(const CopyArgs& a, hipStream_t s) {
+  uint32_t parts = 0;
+  uint64_t most = 0;
+  CopyArgs c{};
+  for (int i = 0; i < 3; ++i) {
+    if (!a.bytes[i]) continue;
+    if (a.bytes[i] % 4u) return hipErrorInvalidValue;
+    c.src[parts] = a.src[i];
+    c.dst[parts] = a.dst[i];
+    c.bytes[parts] = a.bytes[i];
+    most = a.bytes[i] > most ? a.bytes[i] : most;
+    ++parts;
+  }
+  if (!parts) return hipSuccess;
+  const uint64_t wgs = (most + 4095u) / 4096u;
+  hipLaunchKernelGGL(k_copy, dim3((uint32_t)(wgs < 256u ? wgs : 256u), parts), dim3(256), 0, s, c);
+  return hipGetLastError();
+}
+
 __global__ __launch_bounds__(256) void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256u) p[i] = v;
 }
