@@ -956,6 +956,14 @@ static int build_bounds(mrl_ctx* ctx, mrl_index* ix) {
   return MRL_OK;
 }
 
+// Every 1 << sample_shift(B)-th block is what the one-query kernel's sampling
+// pass scores (at most 256 of the B blocks).
+static uint32_t sample_shift(uint64_t B) {
+  uint32_t s = 0;
+  while (((B + (1ull << s) - 1) >> s) > 256) ++s;
+  return s;
+}
+
 // Pass schedule (the same for every K).  When the index has more than 256
 // blocks, a sampling pass first scores every S0-th block (S0 the smallest
 // power of two leaving at most 256 blocks), with no threshold; the final pass
@@ -970,8 +978,7 @@ static int get_levels(mrl_index* ix, uint32_t K, LevelPlan** out) {
   }
   const uint64_t B = ix->n_blocks;
   LevelPlan lp;
-  uint32_t s0 = 0;
-  while (((B + (1ull << s0) - 1) >> s0) > 256) ++s0;
+  const uint32_t s0 = sample_shift(B);
   if (s0 > 0) {
     Pass p;
     p.shift = s0;
@@ -1365,12 +1372,32 @@ static bool excl_ok(const PassBuffers& pb, uint32_t n_q, const ScanParams& sp) {
 // k_select emits the top K (and flags a query whose floor left fewer than K
 // candidates).  rerun_safe: the final pass alone at the safe floor k_select
 // kept (rank K).  Caller holds the context lock.
+// Block bounds apply to scans whose score is the code-space dot product the
+// bounds were built for: the RaBitQ mid-band, an S1 stage, and pruning on.
+static bool bounds_ok(const mrl_index* ix, const mrl_plans* plans, const ScanParams& sp, const PassBuffers& pb) {
+  return pb.block_lists && ix->n_cl != 0 && plans->mid_codec == MRL_MID_RABITQ &&
+         (sp.strata == MRL_STRATA_L1_RABITQ || sp.strata == MRL_STRATA_FULL64B) && !sp.exhaustive;
+}
+
 // The MFMA-bounded path serves batches under the settings where the
 // reference's top K is the top K by full score (the conditions tight_coef()
-// checks on the device) and the RaBitQ mid-band.
-static bool mma_ok(const mrl_plans* plans, uint32_t n_q, const ScanParams& sp, const PassBuffers& pb) {
-  return pb.cand_lower && n_q >= (uint32_t)kMmaMinQ && plans->mid_codec == MRL_MID_RABITQ &&
-         sp.strata != MRL_STRATA_L0_ONLY && sp.alpha >= 1.0f && sp.w_s4 >= 0.0f && 2.4f * sp.w_s4 <= sp.alpha;
+// checks on the device) and the RaBitQ mid-band; of fewer than kMmaMinQ
+// queries those whose queries x blocks pay for its launches, and every batch
+// over block lists whose clusters the one-query kernel's sample misses.
+// That sample then leaves a floor too low for the lists to skip much, and
+// candidate lists overflow into dense re-runs, where the MFMA path's second
+// stage samples within the clusters its first stage finds.  The line: fewer
+// than two sampled blocks per cluster (us per call, one-query kernel / MFMA
+// path, one query: 8.8M vectors in 1,000 clusters 4,165 / 122, 1M in 400
+// 418 / 116, 400K in 400 229 / 112; 1M in 50 74 / 114, 400K in 50 75 / 107).
+static bool mma_ok(const mrl_index* ix, const mrl_plans* plans, uint32_t n_q, const ScanParams& sp,
+                   const PassBuffers& pb) {
+  if (!pb.cand_lower || plans->mid_codec != MRL_MID_RABITQ || sp.strata == MRL_STRATA_L0_ONLY || !(sp.alpha >= 1.0f) ||
+      !(sp.w_s4 >= 0.0f) || !(2.4f * sp.w_s4 <= sp.alpha))
+    return false;
+  const uint64_t B = ix->n_blocks;
+  return n_q >= (uint32_t)kMmaMinQ || (n_q >= 2u && n_q * B >= kMmaMinPairs) ||
+         (bounds_ok(ix, plans, sp, pb) && B < (2ull << sample_shift(B)) * ix->n_cl && B > 256);
 }
 
 // Sampling stages of the MFMA path: blocks b = pos << shift, pos < n_pos.
@@ -1422,13 +1449,6 @@ static std::vector<MmaStage> mma_stages(uint64_t B, uint32_t n_q, uint32_t K, ui
   const uint32_t s2 = B >= 32ull * K && s1 >= 7 ? 6u : 5u;
   if (s1 >= s2 + 1) st.push_back(MmaStage{s2, (uint32_t)((B + (1ull << s2) - 1) >> s2)});
   return st;
-}
-
-// Block bounds apply to scans whose score is the code-space dot product the
-// bounds were built for: the RaBitQ mid-band, an S1 stage, and pruning on.
-static bool bounds_ok(const mrl_index* ix, const mrl_plans* plans, const ScanParams& sp, const PassBuffers& pb) {
-  return pb.block_lists && ix->n_cl != 0 && plans->mid_codec == MRL_MID_RABITQ &&
-         (sp.strata == MRL_STRATA_L1_RABITQ || sp.strata == MRL_STRATA_FULL64B) && !sp.exhaustive;
 }
 
 // Scratch of the block selection of one scan, in the index (grown on demand):
@@ -1735,7 +1755,7 @@ static int enqueue_scan(mrl_ctx* ctx, mrl_index* ix, const mrl_plans* plans, uin
                         unsigned long long* stats, bool rerun_safe = false) {
   // A pending plan build of one query goes into its sampling pass (the fused
   // k_scan); otherwise the plans are built first.
-  const bool mma = mma_ok(plans, n_q, sp, pb);
+  const bool mma = mma_ok(ix, plans, n_q, sp, pb);
   const bool fuse = plans->pending && n_q == 1 && plans_first == 0 && plans->n_q == 1 && !rerun_safe &&
                     lp.passes.size() > 1 && sp.strata != MRL_STRATA_L0_ONLY && plans->dims <= (uint32_t)kFuseMaxDims &&
                     !mma;
@@ -1906,7 +1926,7 @@ static int enqueue_scan_into(mrl_ctx* ctx, const mrl_index* index, const mrl_pla
   LevelPlan* lp;
   if ((rc = get_levels(ix, K, &lp))) return rc;
   const PassBuffers pb = results_buffers(res);
-  *sampled = mma_ok(plans, plans->n_q, sp, pb) ? !mma_stages(ix->n_blocks, plans->n_q, K, 0u).empty()
+  *sampled = mma_ok(ix, plans, plans->n_q, sp, pb) ? !mma_stages(ix->n_blocks, plans->n_q, K, 0u).empty()
                                                : lp->passes.size() > 1;
   res->floor_kind.assign(plans->n_q, *sampled ? 1 : 0);
   return enqueue_scan(ctx, ix, plans, 0, plans->n_q, sp, K, *lp, pb, res->d_stats);
@@ -2459,7 +2479,7 @@ extern "C" int mrl_scan_noalloc(mrl_ctx* ctx, const mrl_index* index, const mrl_
   LevelPlan* lp;
   if ((rc = get_levels(ix, K, &lp))) return rc;
   const bool sampled =
-      mma_ok(plans, n_q, sp, pb) ? !mma_stages(ix->n_blocks, n_q, K, 0u).empty() : lp->passes.size() > 1;
+      mma_ok(ix, plans, n_q, sp, pb) ? !mma_stages(ix->n_blocks, n_q, K, 0u).empty() : lp->passes.size() > 1;
   if ((rc = enqueue_scan(ctx, ix, plans, 0, n_q, sp, K, *lp, pb, nullptr))) return rc;
   // without a sampling pass no query can be flagged
   if (sampled && (rc = enqueue_gated_rerun(ctx, ix, plans, n_q, sp, K, pb))) return rc;

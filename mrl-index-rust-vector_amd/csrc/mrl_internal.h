@@ -157,7 +157,15 @@ constexpr int kRecLev0 = 0, kRecLev1 = 1, kRecS1 = 2, kRecS4Meta = 3;
 constexpr int kMmaSteps = 17;   // K-steps of a tile: prefix 4, S1 8, S4 4, error columns 1
 constexpr int kMmaQ = 64;       // queries per workgroup (two 32-query tiles per wave)
 constexpr int kMmaWaves = 8;    // waves per MFMA scan workgroup (four waves per SIMD)
-constexpr int kMmaMinQ = 8;     // batches of at least this many queries take the MFMA path
+// Batches of at least kMmaMinQ queries take the MFMA path, and smaller ones of
+// two or more once queries x blocks reach kMmaMinPairs: its launches cost
+// 30-40 us more than the one-query kernel's, whose passes cost 8.7 us per
+// query and 1M vectors (us per call, one-query kernel / MFMA path: 1M vectors
+// 5 queries 96.5 / 107, 6 queries 117 / 115, 7 queries 129 / 115; 8.8M vectors
+// 1 query 143 / 222, 2 queries 290 / 234, 4 queries 364 / 243, 7 queries
+// 548 / 253; 131K vectors 7 queries 74 / 95).
+constexpr int kMmaMinQ = 8;
+constexpr uint64_t kMmaMinPairs = 100000;
 constexpr int kTileQ = 8;       // queries per tile of the batched exact kernel (k_scan_tile)
 constexpr int kFuseMaxDims = 1024;  // queries up to this many dims may build their plan inside the sampling pass
 // Per-query constants written by k_mma_prep (floats).

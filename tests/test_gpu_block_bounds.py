@@ -11,6 +11,8 @@ in the header bytes the reference's scan never reads, src/block.rs:37-43).
   still return the oracle's top K: the one-query kernel, k_scan_tile and the
   MFMA path.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -190,3 +192,79 @@ def test_cluster_grouped_mma_two_stage_lists(device):
     assert res.stats.blocks < 0.5 * nb * nq, (res.stats.blocks, nb * nq)
     assert res.stats.reruns_dense == 0
     ix.close()
+
+
+def _scan_route(dev, ix, plan, cfg, lo=None, hi=None):
+    """The scan's result and whether it took the MFMA path (its k_finish ran)."""
+    L = m._lib.lib
+    kt = (m._lib.KernelTimeC * 256)()
+    n = C.c_uint32()
+    m._lib.check(L.mrl_ctx_set_profiling(dev.handle, 1))
+    r = m.scan_batch(ix, plan, cfg, lo, hi)
+    m._lib.check(L.mrl_ctx_profile_collect(dev.handle, kt, 256, C.byref(n)))
+    m._lib.check(L.mrl_ctx_set_profiling(dev.handle, 0))
+    return r, any(kt[i].kind == m._lib.KERNEL_FINISH for i in range(min(n.value, 256)))
+
+
+@pytest.mark.parametrize("n_clusters,per,mma", [(300, 128, True), (20, 1920, False)])
+@pytest.mark.parametrize("nq", [1, 2, 7])
+def test_small_batches_over_block_lists(n_clusters, per, mma, nq):
+    """Fewer than 8 queries over block lists: the MFMA path where the
+    one-query kernel's sample holds fewer than two blocks per cluster, that
+    kernel otherwise; the oracle's lists either way, at every option the
+    rule looks at."""
+    dev = m.Device(0)
+    rows, cl = clustered_rows(n_clusters, n_clusters, per, 192)
+    blocks = m.encode_corpus_clustered(rows, cl, 8)
+    ix = m.DeviceIndex.upload(blocks, dev)
+    rng = np.random.default_rng(nq)
+    qs = (rows[rng.integers(0, rows.shape[0], nq)] + 0.01 * rng.standard_normal((nq, 192))).astype(np.float32)
+    plan = m.QueryPlan.from_query(qs, 192, dev)
+    n = rows.shape[0]
+    for k, depth, lo, hi in ((64, 2, None, None), (256, 1, None, None), (1000, 2, n // 4, n // 2), (1, 2, None, None)):
+        cfg = m.ScanConfig(shortlist_cand=k, strata_depth=m.StrataDepth(depth))
+        r, took = _scan_route(dev, ix, plan, cfg, lo, hi)
+        assert took == mma, (k, depth)
+        for qi in range(nq):
+            rid, rsc = ora.scan_blocks(blocks, ora.plan_build(qs[qi], 192), ora.scan_config(k, depth=depth), lo, hi)
+            c = int(r.counts[qi])
+            assert c == len(rid)
+            assert_topk_equal(r.ids[qi, :c], r.scores[qi, :c], rid, rsc, k, f"k={k} depth={depth} q={qi}")
+    cfg = m.ScanConfig(shortlist_cand=64, exhaustive=True)  # no lists: the one-query kernel
+    assert not _scan_route(dev, ix, plan, cfg)[1]
+    for o in (plan, ix, dev):
+        o.close()
+
+
+def test_small_batches_over_many_blocks():
+    """Two and more queries take the MFMA path once queries x blocks reach its
+    line, and return what each query returns alone."""
+    dev = m.Device(0)
+    rng = np.random.default_rng(3)
+    n_blocks = 50_000
+    blocks = rng.integers(0, 256, (n_blocks, 4096), dtype=np.uint8)
+    blocks[:, :64] = 0
+    meta = np.zeros((n_blocks * 64, 7), dtype=np.uint8)
+    meta[:, 0:2] = rng.uniform(0.1, 0.3, n_blocks * 64).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    meta[:, 4:6] = rng.uniform(0.7, 1.0, n_blocks * 64).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    meta[:, 6] = rng.integers(150, 250, n_blocks * 64)
+    blocks[:, 64:512] = meta.reshape(n_blocks, 448)
+    ix = m.DeviceIndex.upload(blocks, dev)
+    fit = m.EdenFit.default_prefix(1)
+    qs = normalized(rng, 3, 768)
+    cfg = m.ScanConfig(shortlist_cand=256)
+    alone = []
+    for q in qs:
+        r, mma = _scan_route(dev, ix, m.QueryPlan.from_query_eden(q, 768, fit, dev), cfg)
+        assert not mma and int(r.counts[0]) == 256
+        alone.append(r)
+    for nq in (2, 3):
+        r, mma = _scan_route(dev, ix, m.QueryPlan.from_query_eden(qs[:nq], 768, fit, dev), cfg)
+        assert mma
+        for i in range(nq):
+            assert np.array_equal(r.ids[i], alone[i].ids[0])
+            assert np.array_equal(r.scores[i].view(np.uint32), alone[i].scores[0].view(np.uint32))
+    small = m.DeviceIndex.upload(blocks[:49_999], dev)
+    assert not _scan_route(dev, small, m.QueryPlan.from_query_eden(qs[:2], 768, fit, dev), cfg)[1]
+    for o in (small, ix, dev):
+        o.close()
