@@ -41,9 +41,18 @@ __device__ __forceinline__ uint32_t f32_to_f16(float f) {
   return out & 0xffffu;
 }
 
+// The workgroup's barrier before signal_status.  A wave waits for its own
+// stores first: __syncthreads() orders them within the workgroup only (it is
+// compiled without a wait for stores), and the signalling thread's release
+// waits for the stores of its own wave.
+__device__ __forceinline__ void signal_barrier() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
 // Stores a query's status in host memory once everything its workgroup wrote
-// is visible there (called by one thread after the workgroup's barrier).  The
-// host polls the word: the wait ends about 5 us before the stream's own
+// is visible there (called by one thread after signal_barrier).  The host
+// polls the word: the wait ends about 5 us before the stream's own
 // completion signal would wake a hipStreamSynchronize (an empty kernel: 8.0
 // against 13.6 us).
 __device__ __forceinline__ void signal_status(uint32_t* status, uint32_t value) {

@@ -2355,7 +2355,7 @@ __global__ __launch_bounds__(kSelThreads) void k_select(SelectArgs a) {
   if (tid < (int)a.nseg) a.seg_count[(uint64_t)q * a.nseg + tid] = 0u;
   if (a.hist)
     for (int i = tid; i < kHistBins; i += kSelThreads) a.hist[(uint64_t)q * kHistBins + i] = 0u;
-  if (a.signal) __syncthreads();  // every thread's outputs before the status
+  if (a.signal) signal_barrier();  // every thread's outputs before the status
   if (tid == 0) {
     // Fewer than K candidates above a floor tighter than the safe one: the
     // top K may lie below it, so the final pass is re-run at the safe floor.

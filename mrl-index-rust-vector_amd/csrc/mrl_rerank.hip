@@ -355,7 +355,7 @@ __global__ __launch_bounds__(kSortThreads) void k_rerank_sort(RerankArgs a) {
     a.out_rows[base + r] = in ? a.row[base + i] : 0ull;
     a.out_scores[base + r] = in ? a.score[base + i] : 0.0f;
   }
-  if (a.signal) __syncthreads();  // every thread's outputs before the status
+  if (a.signal) signal_barrier();  // every thread's outputs before the status
   if (tid == 0) {
     const uint32_t status = s_bad | (a.scan_status ? (a.scan_status[q] & 7u) << 8 : 0u);
     if (a.out_counts) a.out_counts[q] = m - s_skip;
