@@ -141,6 +141,13 @@ __device__ __forceinline__ uint32_t count_of(const RerankArgs& a, uint32_t q) {
   return a.counts ? a.counts[q] : a.stride;
 }
 
+// Makes this wave's LDS writes visible to its own later reads.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Candidate c of query q -> store row.  *ok false: no row to score (*row says why).
 __device__ __forceinline__ void resolve_row(const RerankArgs& a, uint32_t q, uint32_t c, uint64_t* row, bool* ok) {
   if (!a.cand) {
@@ -249,30 +256,118 @@ __global__ __launch_bounds__(kScoreThreads) void k_score768(RerankArgs a, uint32
   }
 }
 
-// fp32 at dims != 768: one lane per candidate, sequential from -0.0.
+// fp32 at dims != 768: sequential sums from -0.0, one lane per candidate.  A
+// wave takes kSeqCand candidates; pieces of kSeqDims dims come in with
+// coalesced loads, one piece ahead of their use, and their products go through
+// the wave's LDS to the lanes that add.  What bounds it: HBM for batches (a
+// lane that reads its own row touches a cache line per 4 bytes loaded), for
+// few candidates the memory latency of a piece, so 16 per wave: more loads in
+// flight per candidate and four times the waves of 64.  WIDE: 16-byte loads,
+// where rows start at 16-byte multiples.  us per mrl_rerank_rows call, one
+// lane reading its own row -> this: 16 queries of 256 rows x 1024 dims
+// 57-64 -> 40, 64 of 256 x 512 60 -> 46.5, 256 of 256 x 1024 167 -> 150 (the
+// rest is the transfer of the lists), one of 64 x 1024 38.4 -> 31.5, 64 of
+// 256 x 1001 (4-byte loads) 103 -> 61.5.
+constexpr uint32_t kSeqCand = 16;
+constexpr uint32_t kSeqDims = 128;
+constexpr uint32_t kSeqStride = kSeqDims + 4;  // LDS row (16 rows' 16-byte reads cover every bank)
+constexpr uint32_t kSeqGroup = kScoreThreads / 64 * kSeqCand;
+template <bool WIDE>
 __global__ __launch_bounds__(kScoreThreads) void k_score_seq(RerankArgs a, uint32_t n_chunks) {
-  __shared__ float s_q[MRL_MAX_DIMS];
+  __shared__ __align__(16) float s_prod[kScoreThreads / 64][kSeqCand * kSeqStride];
   const uint32_t q = blockIdx.x / n_chunks;
-  const uint32_t base = (blockIdx.x % n_chunks) * kScoreThreads;
+  const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+  const uint32_t base = (blockIdx.x % n_chunks) * kSeqGroup + w * kSeqCand;
   const uint32_t cnt = count_of(a, q);
-  if (base >= cnt) return;
+  if (base >= cnt) return;  // (the wave's; no workgroup barrier follows)
   const uint32_t dims = a.dims;
   const float* qv = a.queries + (uint64_t)q * dims;
-  for (uint32_t i = threadIdx.x; i < dims; i += kScoreThreads) s_q[i] = qv[i];
-  __syncthreads();
-  const uint32_t c = base + threadIdx.x;
-  if (c >= cnt) return;
-  uint64_t row;
-  bool ok;
-  resolve_row(a, q, c, &row, &ok);
-  float s = -0.0f;
-  if (ok) {
-    const float* r = static_cast<const float*>(a.data) + row * dims;
-    for (uint32_t i = 0; i < dims; ++i) s = s + s_q[i] * r[i];
+  const uint32_t c = base + (lane & (kSeqCand - 1u));
+  uint64_t row = kRowBad;
+  bool ok = false;
+  if (c < cnt) resolve_row(a, q, c, &row, &ok);
+  const float* data = static_cast<const float*>(a.data);
+  const unsigned long long off = ok ? row * dims : ~0ull;
+  // element u of a lane: candidate kStep u + lane / kLanes, kPer dims from lane % kLanes
+  constexpr uint32_t kPer = WIDE ? 4u : 2u;
+  constexpr uint32_t kLanes = kSeqDims / kPer, kStep = 64u / kLanes, kLoads = kSeqCand / kStep;
+  const uint32_t d = WIDE ? 4u * (lane & (kLanes - 1u)) : lane;  // not WIDE: dims d and d + 64
+  float* sp = s_prod[w];
+  float v[kLoads][kPer], qd[kPer];
+  unsigned long long wide_off[WIDE ? kLoads : 1];
+  if constexpr (WIDE) {
+#pragma unroll
+    for (uint32_t u = 0; u < kLoads; ++u) wide_off[u] = __shfl(off, (int)(kStep * u + lane / kLanes));
   }
-  const uint64_t o = (uint64_t)q * a.stride + c;
-  a.score[o] = ok ? s : 0.0f;
-  a.row[o] = row;
+  auto load = [&](uint32_t at) {
+#pragma unroll
+    for (uint32_t e = 0; e < kPer; ++e) {
+      const uint32_t i = at + d + (WIDE ? e : 64u * e);
+      qd[e] = i < dims ? qv[i] : 0.0f;
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kLoads; ++u) {
+      unsigned long long o;
+      if constexpr (WIDE)
+        o = wide_off[u];
+      else  // one candidate for the whole wave
+        o = (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(off >> 32), (int)u) << 32 |
+            (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)off, (int)u);
+      const float* r = data + o + at + d;
+      const uint32_t left = o != ~0ull && at + d < dims ? dims - at - d : 0u;  // of the row, from r on
+      if (WIDE) {
+        float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (left) f = *reinterpret_cast<const float4*>(r);
+        v[u][0] = f.x;
+        v[u][1] = f.y;
+        v[u][kPer - 2] = f.z;
+        v[u][kPer - 1] = f.w;
+      } else {
+#pragma unroll
+        for (uint32_t e = 0; e < kPer; ++e) v[u][e] = 64u * e < left ? r[64u * e] : 0.0f;
+      }
+    }
+  };
+  float s = -0.0f;
+  load(0);
+  for (uint32_t at = 0; at < dims; at += kSeqDims) {
+#pragma unroll
+    for (uint32_t u = 0; u < kLoads; ++u) {
+      float* o = sp + (kStep * u + lane / kLanes) * kSeqStride + d;
+      if (WIDE)
+        *reinterpret_cast<float4*>(o) = make_float4(qd[0] * v[u][0], qd[1] * v[u][1], qd[kPer - 2] * v[u][kPer - 2],
+                                                    qd[kPer - 1] * v[u][kPer - 1]);
+      else
+#pragma unroll
+        for (uint32_t e = 0; e < kPer; ++e) o[64u * e] = qd[e] * v[u][e];
+    }
+    wave_lds_sync();
+    if (at + kSeqDims < dims) load(at + kSeqDims);
+    if (lane < kSeqCand) {
+      const float* p = sp + lane * kSeqStride;
+      const uint32_t nd = dims - at < kSeqDims ? dims - at : kSeqDims;
+      uint32_t t = 0;
+      for (; t + 16u <= nd; t += 16u) {
+        float4 f[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) f[u] = *reinterpret_cast<const float4*>(p + t + 4 * u);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          s = s + f[u].x;
+          s = s + f[u].y;
+          s = s + f[u].z;
+          s = s + f[u].w;
+        }
+      }
+      for (; t < nd; ++t) s = s + p[t];
+    }
+    wave_lds_sync();  // the sums are done before the next products
+  }
+  if (lane < kSeqCand && c < cnt) {
+    const uint64_t o = (uint64_t)q * a.stride + c;
+    a.score[o] = ok ? s : 0.0f;
+    a.row[o] = row;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -612,8 +707,12 @@ hipError_t launch_rerank(const RerankArgs& a, hipStream_t s, const LaunchEvents&
     else
       launch(k_score768<MRL_RERANK_INT8>, grid, dim3(kScoreThreads), s, ev_score, a, n_chunks);
   } else {
-    const uint32_t n_chunks = (a.stride + kScoreThreads - 1) / kScoreThreads;
-    launch(k_score_seq, dim3(n_chunks * a.n_q), dim3(kScoreThreads), s, ev_score, a, n_chunks);
+    const uint32_t n_chunks = (a.stride + kSeqGroup - 1) / kSeqGroup;
+    const dim3 grid(n_chunks * a.n_q);
+    if (a.dims % 4u == 0 && (reinterpret_cast<uintptr_t>(a.data) & 15u) == 0)
+      launch(k_score_seq<true>, grid, dim3(kScoreThreads), s, ev_score, a, n_chunks);
+    else
+      launch(k_score_seq<false>, grid, dim3(kScoreThreads), s, ev_score, a, n_chunks);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

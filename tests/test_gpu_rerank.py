@@ -110,6 +110,28 @@ def test_rerank_generic_dims_fp32(device, dims):
         m.RerankStore.create(rows, m.RerankPrecision.FP16, device)  # fp16 / int8 need 768 dims
 
 
+@pytest.mark.parametrize("dims", [1, 3, 4, 63, 64, 65, 127, 128, 129, 132, 254, 256, 516, 1024, 2050])
+def test_rerank_generic_dims_pieces(device, dims):
+    """Edges of the generic scoring kernel's pieces (16 candidates a wave, 64 a
+    workgroup, 128 dims), with 4-byte and 16-byte loads; the rows at the
+    store's end among the candidates."""
+    rng = np.random.default_rng(2000 + dims)
+    rows = rng.standard_normal((67, dims)).astype(np.float32)
+    rows[5] = 0.0
+    rows[6] = -rows[7]
+    counts = np.array([131, 64, 65, 63, 17, 16, 15, 1, 0], dtype=np.uint32)
+    q = rng.standard_normal((counts.size, dims)).astype(np.float32)
+    cand = rng.integers(0, 67, (counts.size, 131)).astype(np.uint64)
+    cand[:, 0] = 66
+    store = m.RerankStore.create(rows, m.RerankPrecision.FP32, device)
+    got_r, got_s = m.rerank_batch(store, q, cand, counts)
+    _check_batch(ora.RERANK_FP32, q, rows, cand, counts, got_r, got_s, f"dims={dims}")
+    cand[1, 63] = 67
+    with pytest.raises(m.MrlError) as e:
+        m.rerank_batch(store, q, cand, counts)
+    assert e.value.code == 1
+
+
 @pytest.mark.parametrize("prec,prec_o", PRECS)
 def test_rerank_ties_keep_input_order(device, prec, prec_o):
     rows = _rows(6, 64)
