@@ -888,8 +888,22 @@ static int build_bounds(mrl_ctx* ctx, mrl_index* ix) {
   const uint64_t B = ix->n_blocks;
   if (!B) return MRL_OK;
   std::vector<uint32_t> h3(B);
-  HIP_TRY(hipMemcpy2DAsync(h3.data(), 4, ix->d_blocks + 12, kBlockBytes, 4, B, hipMemcpyDeviceToHost, ctx->stream));
-  HIP_TRY(hipStreamSynchronize(ctx->stream));
+  {
+    const uint64_t step = 1u << 15;  // blocks at a time
+    const size_t bytes = (size_t)std::min(B, step) * 4;
+    uint32_t* h = reinterpret_cast<uint32_t*>(ctx->pin_pool.take(bytes));
+    if (!h) return fail(MRL_ERR_OUT_OF_MEMORY, "block headers");
+    hipError_t e = hipSuccess;
+    for (uint64_t b = 0; b < B && e == hipSuccess; b += step) {
+      const uint32_t n = (uint32_t)std::min(step, B - b);
+      e = launch_header_words(ix->d_blocks + b * kBlockBytes, n, h, ctx->stream);
+      const hipError_t es = hipStreamSynchronize(ctx->stream);
+      if (e == hipSuccess) e = es;
+      if (e == hipSuccess) memcpy(h3.data() + b, h, (size_t)n * 4);
+    }
+    ctx->pin_pool.give(h, bytes);
+    if (e != hipSuccess) return fail(MRL_ERR_HIP, std::string("block headers: ") + hipGetErrorString(e));
+  }
   std::map<uint32_t, uint32_t> dense;
   std::vector<uint32_t> bcl(B, ~0u);
   for (uint64_t b = 0; b < B; ++b)

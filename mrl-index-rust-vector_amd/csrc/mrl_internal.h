@@ -572,6 +572,8 @@ struct CopyArgs {
   uint64_t bytes[3];
 };
 hipError_t launch_copy(const CopyArgs& a, hipStream_t s);
+// Header dword 3 of n blocks into mapped host memory.
+hipError_t launch_header_words(const uint8_t* blocks, uint32_t n, uint32_t* out, hipStream_t s);
 // Sets n words at p to v (a kernel, so that a caller may capture it in a graph).
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
 // Reads n uint4 at p (evicts the caches; the loads are kept alive by a store

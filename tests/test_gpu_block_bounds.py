@@ -268,3 +268,26 @@ def test_small_batches_over_many_blocks():
     assert not _scan_route(dev, small, m.QueryPlan.from_query_eden(qs[:2], 768, fit, dev), cfg)[1]
     for o in (small, ix, dev):
         o.close()
+
+
+@pytest.mark.parametrize("n_blocks", [1, 255, 257, 32767, 32768, 32770])
+def test_flagged_blocks_of_large_indexes(device, n_blocks):
+    """The headers are read in pieces of 32,768 blocks: every flagged block, and
+    no other, has bounds."""
+    rng = np.random.default_rng(n_blocks)
+    blocks = np.tile(rng.integers(0, 256, (64, 4096), dtype=np.uint8), ((n_blocks + 63) // 64, 1))[:n_blocks].copy()
+    blocks[:, :64] = 0
+    meta = np.zeros((64, 7), dtype=np.uint8)
+    meta[:, 0:2] = rng.uniform(0.1, 0.3, 64).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    meta[:, 4:6] = rng.uniform(0.7, 1.0, 64).astype(np.float16).view(np.uint8).reshape(-1, 2)
+    meta[:, 6] = 200
+    blocks[:, 64:512] = meta.reshape(1, 448)
+    flagged = np.arange(n_blocks) % 3 == 0
+    flagged[-1] = True
+    blocks[:, 12] = np.arange(n_blocks) % 11
+    blocks[:, 14] = flagged
+    ix = m.DeviceIndex.upload(blocks, device)
+    plan = m.QueryPlan.from_query(normalized(rng, 2, 192), 192, device)
+    bnd = m.index_block_bounds(ix, plan, m.ScanConfig())
+    assert np.array_equal(np.isnan(bnd), np.broadcast_to(~flagged, (2, n_blocks)))
+    ix.close()
